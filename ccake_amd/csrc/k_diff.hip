@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kWave) void k_diff_slice(const double* __restrict__
                                                       const int32_t* __restrict__ skey,
                                                       const int32_t* __restrict__ cell_off,
                                                       const Grid* __restrict__ gridp, int n,
-                                                      double rc2, double rcs, double hinv2, int nslices,
+                                                      double rc2, double rcs, double m4h, double m2h, int nslices,
                                                       double* __restrict__ part, int npad)
 {
   const Grid g0 = *gridp;
@@ -138,13 +138,11 @@ __global__ __launch_bounds__(kWave) void k_diff_slice(const double* __restrict__
 
   for_segments(act, myrow, xa, ya, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    for_spans_slice(g, cell_off, seg, rcs, slice, nslices, in, [&](int j0, int j1) {
-      walk_records<15, kCandD, 1>(cand, xa, ya, j0, j1, [&](const double* c, double dx, double dy, int j, bool valid) {
-        const double r2 = dist2_nocontract(dx, dy);
-        if (kSkipEmpty && wave_none(valid && r2 <= rc2)) return;
-        double q, iq;
-        q_and_inverse(r2, hinv2, q, iq);
-        const double gm = valid ? c[2] * spline_g(q, iq) : 0.0;
+    const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
+    for_spans_slice<kCandD, false>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
+      walk_records<15, kCandD, 1>(cand, xs, ya, cur,
+                               [&](const double* c, double dx, double dy, double r2) {
+        const double gm = c[2] * spline_g2(r2, m4h, m2h);
         const double wx = gm * dx, wy = gm * dy;
         acc[0] += wx; acc[1] += wy;
         #pragma unroll
@@ -157,8 +155,9 @@ __global__ __launch_bounds__(kWave) void k_diff_slice(const double* __restrict__
     });
   });
 
+  const double h2 = -1.0 / m2h;                // spline_g2's factor
   double* p = part + (size_t)slice * kDiffAcc * npad + k;
-  for (int q = 0; q < kDiffAcc; ++q) p[(size_t)q * npad] = acc[q];
+  for (int q = 0; q < kDiffAcc; ++q) p[(size_t)q * npad] = h2 * acc[q];
 }
 
 template <int S>
@@ -241,7 +240,7 @@ int launch_diff_grad(ccake_event* ev)
   const double rc = 2.0 * h;
   const int ntiles = (n + kTile - 1) / kTile;
   hipLaunchKernelGGL(k_diff_slice, dim3(ntiles * ev->nslices), dim3(kWave), 0, ev->stream, ev->cand_d, ev->skey,
-                     ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), 1.0 / (h * h), ev->nslices, ev->part,
+                     ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), -0.25 / h, -0.5 / h, ev->nslices, ev->part,
                      ev->npad);
   if (hipGetLastError() != hipSuccess) return CCAKE_ERR_HIP;
   const double C = -0.5 * (15.0 / (7.0 * kPi)) / pow(h, 4);

@@ -14,66 +14,99 @@
 // applies the owner terms once at the end.
 #include "pair_common.h"
 #include "grad_sum.h"
+#include <type_traits>
 
 namespace ccake {
 
 // The walk of one (tile, slice) unit: slice `slice` of `nslices` of the
-// tile's candidates, one wave; fin(acc) receives the neighbour-side sums.
+// tile's candidates, one wave; fin(acc) receives the neighbour-side sums of
+// m_b grad W / C, summed as spline_g2 m_b rel and scaled by its 2 h at the end
+// (KEEP: with the arithmetic of q_and_inverse and spline_g, keep_order).
 // BULK false: the event's bulk pressure is zero on every particle (zeta = 0
 // and no initial bulk, checked at initialize), so the grad Pi sums are the
 // exact zeros the full walk would give and are not accumulated.
-template <bool SHEAR, bool BULK, class Fin>
+// Bound: the FP64 vector unit (80 % busy), 38 instructions per candidate and
+// wave: the 20 sums, 5 for the offsets and r^2, 13 for the kernel.  FP64
+// matrix instructions run in the same unit at the same rate (16x16x4: 65
+// cycles, a vector instruction 4), so the sums stay on the vector side.
+// 188,250 particles (479M pairs): 1.30 ms per launch with 50 instructions
+// and no request ahead, 0.96 ms now.
+template <bool SHEAR, bool BULK, bool KEEP, class Fin>
 __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const int32_t* __restrict__ skey,
                                           const int32_t* __restrict__ cell_off, const Grid* __restrict__ gridp,
-                                          int n, double rc2, double rcs, double hinv2, int tile, int slice,
+                                          int n, double rc2, double rcs, double hinv2, double m4h, double m2h, int tile, int slice,
                                           int nslices, Fin&& fin)
 {
-  constexpr int NACC = grad_nacc<SHEAR>();
-  const Grid g0 = *gridp;
+  const Grid& g0 = *gridp;
   const int lane = threadIdx.x & (kWave - 1);
   const int k = tile * kTile + lane;
   const bool act = k < n;
   const int kk = act ? k : 0;
   const double* me = cand + (size_t)kk * kCandG;
   const double xa = me[0], ya = me[1];
-  const double vax = me[6], vay = me[7];
   const int myrow = act ? skey[kk] / g0.stride : INT_MAX;
 
-  double acc[NACC];
-  for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
+  // the 12 sums of grad_nacc<false>, then pi^{0x} w (2), pi^{0y} w (2) and
+  // the two of pi^{ij} w_i; KEEP: the sums of grad_nacc<SHEAR> themselves
+  constexpr int NW = SHEAR ? (KEEP ? 17 : 18) : 12;
+  const double vax = me[6], vay = me[7];
+  double acc[NW];
+  #pragma unroll
+  for (int q = 0; q < NW; ++q) acc[q] = 0.0;
 
   for_segments(act, myrow, xa, ya, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    // lanes of other cell rows sit this segment's walk out
-    for_spans_slice(g, cell_off, seg, rcs, slice, nslices, in, [&](int j0, int j1) {
-      // Candidate records are wave-uniform (scalar loads into SGPRs); the
-      // shear record is too large to hold two steps of two in SGPRs.
+    const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
+    for_spans_slice<kCandG, KEEP>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
       constexpr int NR = SHEAR ? 13 : 8;
-      walk_records<NR, kCandG, SHEAR ? 1 : 2>(cand, xa, ya, j0, j1,
-                                              [&](const double* c, double dx, double dy, int j, bool valid) {
-        const double r2 = dist2_nocontract(dx, dy);
-        if (kSkipEmpty && wave_none(valid && r2 <= rc2)) return;
-        double q, iq;
-        q_and_inverse(r2, hinv2, q, iq);
-        const double gm = valid ? c[2] * spline_g(q, iq) : 0.0;
+      walk_records<NR, kCandG, 1>(cand, xs, ya, cur,
+                               [&](const double* c, double dx, double dy, double r2) {
+        double gm;
+        if (KEEP) {
+          double q, iq;
+          q_and_inverse(r2, hinv2, q, iq);
+          gm = c[2] * spline_g(q, iq);
+        } else {
+          gm = c[2] * spline_g2(r2, m4h, m2h);
+        }
         const double wx = gm * dx, wy = gm * dy;
-        acc[0] += wx; acc[1] += wy;                    // sum m_b grad W / C
+        acc[0] += wx; acc[1] += wy;                    // sum m_b grad W
         acc[2] += c[3] * wx; acc[3] += c[3] * wy;      // p_b / sl_b^2
         acc[4] += c[4] * wx; acc[5] += c[4] * wy;      // e_b
         if (BULK) { acc[6] += c[5] * wx; acc[7] += c[5] * wy; }   // Pi_b / sl_b^2
         acc[8] += c[6] * wx; acc[9] += c[7] * wx;      // v_b d_x W
         acc[10] += c[6] * wy; acc[11] += c[7] * wy;    // v_b d_y W
-        if (SHEAR) {
+        if (SHEAR && KEEP) {
           const double cv = wx * vax + wy * vay;
           acc[SHEAR ? 12 : 0] += cv;
           acc[SHEAR ? 13 : 0] += cv * c[SHEAR ? 8 : 0]; acc[SHEAR ? 14 : 0] += cv * c[SHEAR ? 9 : 0];
           acc[SHEAR ? 15 : 0] += wx * c[SHEAR ? 10 : 0] + wy * c[SHEAR ? 11 : 0];
           acc[SHEAR ? 16 : 0] += wx * c[SHEAR ? 11 : 0] + wy * c[SHEAR ? 12 : 0];
+        } else if (SHEAR) {
+          acc[SHEAR ? 12 : 0] += c[SHEAR ? 8 : 0] * wx; acc[SHEAR ? 13 : 0] += c[SHEAR ? 8 : 0] * wy;
+          acc[SHEAR ? 14 : 0] += c[SHEAR ? 9 : 0] * wx; acc[SHEAR ? 15 : 0] += c[SHEAR ? 9 : 0] * wy;
+          acc[SHEAR ? 16 : 0] += c[SHEAR ? 10 : 0] * wx; acc[SHEAR ? 16 : 0] += c[SHEAR ? 11 : 0] * wy;
+          acc[NW - 1] += c[SHEAR ? 11 : 0] * wx; acc[NW - 1] += c[SHEAR ? 12 : 0] * wy;
         }
       });
     });
   });
-  fin(acc);
+  if (!KEEP) {
+    const double h2 = -1.0 / m2h;
+    #pragma unroll
+    for (int q = 0; q < NW; ++q) acc[q] *= h2;
+  }
+  if (SHEAR && !KEEP) {
+    // w . v_a and (w . v_a) pi^{0i}_b / sl_b^2, v_a being constant over b
+    const double out[17] = { acc[0], acc[1], acc[2], acc[3], acc[4], acc[5], acc[6], acc[7], acc[8], acc[9], acc[10],
+                             acc[11], vax * acc[0] + vay * acc[1],
+                             vax * acc[SHEAR ? 12 : 0] + vay * acc[SHEAR ? 13 : 0],
+                             vax * acc[SHEAR ? 14 : 0] + vay * acc[SHEAR ? 15 : 0],
+                             acc[SHEAR ? 16 : 0], acc[NW - 1] };
+    fin(out);
+  } else {
+    fin(acc);
+  }
 }
 
 // Pair part: one single-wave workgroup per (tile, slice) unit walks its
@@ -84,14 +117,14 @@ __global__ __launch_bounds__(kWave) void k_grad_slice(const double* __restrict__
                                                       const int32_t* __restrict__ skey,
                                                       const int32_t* __restrict__ cell_off,
                                                       const Grid* __restrict__ gridp, int n,
-                                                      double rc2, double rcs, double hinv2, int nslices,
+                                                      double rc2, double rcs, double hinv2, double m4h, double m2h, int nslices,
                                                       double* __restrict__ part, int npad)
 {
   constexpr int NACC = grad_nacc<SHEAR>();
   const int unit = xcd_tile(blockIdx.x, gridDim.x);
   const int tile = unit / nslices;
   const int slice = unit - tile * nslices;
-  grad_walk<SHEAR, BULK>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, tile, slice, nslices,
+  grad_walk<SHEAR, BULK, false>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, m2h, tile, slice, nslices,
                          [&](const double* acc) {
     double* p = part + (size_t)slice * NACC * npad + tile * kTile + threadIdx.x;
     for (int q = 0; q < NACC; ++q) p[(size_t)q * npad] = acc[q];
@@ -103,31 +136,40 @@ __global__ __launch_bounds__(kWave) void k_grad_slice(const double* __restrict__
 // and stored as the sums of a single slice, so the sum pass reads NACC
 // values per particle instead of W * NACC and no partial sum of a slice
 // goes through HBM.
-template <bool SHEAR, bool BULK, int W>
+template <bool SHEAR, bool BULK, int W, bool KEEP = false>
 __global__ __launch_bounds__(kWave * W) void k_grad_tile(const double* __restrict__ cand,
                                                          const int32_t* __restrict__ skey,
                                                          const int32_t* __restrict__ cell_off,
                                                          const Grid* __restrict__ gridp, int n,
-                                                         double rc2, double rcs, double hinv2,
+                                                         double rc2, double rcs, double hinv2, double m4h, double m2h,
                                                          double* __restrict__ part, int npad)
 {
-  constexpr int NACC = grad_nacc<SHEAR>();
-  __shared__ double red[W][NACC][kWave];
+  // the sums go through LDS in two halves: 18 KB a tile of 4 waves instead of
+  // 35, so that LDS does not hold the CU below its 6 waves per SIMD
+  constexpr int NACC = grad_nacc<SHEAR>(), HALF = (NACC + 1) / 2;
+  __shared__ double red[W][HALF][kWave];
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int slice = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // wave-uniform
   const int lane = threadIdx.x & (kWave - 1);
-  grad_walk<SHEAR, BULK>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, tile, slice, W, [&](const double* acc) {
+  grad_walk<SHEAR, BULK, KEEP>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, m2h, tile, slice, W,
+                               [&](const double* acc) {
     #pragma unroll
-    for (int q = 0; q < NACC; ++q) red[slice][q][lane] = acc[q];
+    for (int h = 0; h < 2; ++h) {
+      if (h) __syncthreads();                    // the first half has been read
+      #pragma unroll
+      for (int q = 0; q < HALF; ++q)
+        if (h * HALF + q < NACC) red[slice][q][lane] = acc[h * HALF + q < NACC ? h * HALF + q : 0];
+      __syncthreads();
+      const int nq = NACC - h * HALF < HALF ? NACC - h * HALF : HALF;
+      for (int t = threadIdx.x; t < nq * kWave; t += kWave * W) {
+        const int q = t / kWave, l = t - q * kWave;
+        double s = 0.0;
+        #pragma unroll
+        for (int w = 0; w < W; ++w) s += red[w][q][l];
+        part[(size_t)(h * HALF + q) * npad + tile * kTile + l] = s;
+      }
+    }
   });
-  __syncthreads();
-  for (int t = threadIdx.x; t < NACC * kWave; t += kWave * W) {
-    const int q = t / kWave, l = t - q * kWave;
-    double s = 0.0;
-    #pragma unroll
-    for (int w = 0; w < W; ++w) s += red[w][q][l];
-    part[(size_t)q * npad + tile * kTile + l] = s;
-  }
 }
 
 // Sum pass: the slices' sums in slice order, scaled by C = kgrad / h^4,
@@ -150,29 +192,34 @@ int launch_grad_pairs(ccake_event* ev)
   const int n = ev->n_live;          // sorted positions of the live events' particles
   const double h = ev->p.hT;
   const double rc = 2.0 * h;
-  const double hinv2 = 1.0 / (h * h);
+  const double hinv2 = 1.0 / (h * h), m4h = -0.25 / h, m2h = -0.5 / h;
   const int ntiles = (n + kTile - 1) / kTile;
   const double rcs = search_radius(ev);
-  // tiles of 4 waves: 1.318 ms per launch on the 200k event against 1.343
-  // with 8 (the smoothing walk prefers 8)
-  const int W = lds_slices(ev) ? 4 : 0;
+  const int W = grad_tile_waves(lds_slices(ev), ntiles, ev->dev->simds);
   if (W) {
     // the tile's slices reduced in LDS: the sum pass sees one slice
     ev->grad_sum_slices = 1;
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kWave * W), 0, ev->stream, ev->cand_g, ev->skey, ev->cell_off,
-                         ev->grid, n, rc * rc, rcs, hinv2, ev->part, ev->npad);
+    auto go = [&](auto kern, int nw) {
+      hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kWave * nw), 0, ev->stream, ev->cand_g, ev->skey, ev->cell_off,
+                         ev->grid, n, rc * rc, rcs, hinv2, m4h, m2h, ev->part, ev->npad);
     };
-    const bool sh = ev->p.using_shear, bu = !ev->no_bulk;
-    if (sh) { if (bu) go(k_grad_tile<true, true, 4>); else go(k_grad_tile<true, false, 4>); }
-    else { if (bu) go(k_grad_tile<false, true, 4>); else go(k_grad_tile<false, false, 4>); }
+    auto waves = [&](auto w, auto keep) {
+      constexpr int V = decltype(w)::value;
+      constexpr bool K = decltype(keep)::value;
+      const bool sh = ev->p.using_shear, bu = !ev->no_bulk;
+      if (sh) { if (bu) go(k_grad_tile<true, true, V, K>, V); else go(k_grad_tile<true, false, V, K>, V); }
+      else { if (bu) go(k_grad_tile<false, true, V, K>, V); else go(k_grad_tile<false, false, V, K>, V); }
+    };
+    if (W >= 2 * kKeepGradWaves && keep_order(ev, ntiles)) waves(std::integral_constant<int, kKeepGradWaves>(), std::true_type());
+    else if (W == 8) waves(std::integral_constant<int, 8>(), std::false_type());
+    else waves(std::integral_constant<int, 4>(), std::false_type());
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
   }
   ev->grad_sum_slices = ev->nslices;
   const dim3 grid(ntiles * ev->nslices), blk(kWave);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, blk, 0, ev->stream, ev->cand_g, ev->skey, ev->cell_off, ev->grid, n, rc * rc,
-                       rcs, hinv2, ev->nslices, ev->part, ev->npad);
+                       rcs, hinv2, m4h, m2h, ev->nslices, ev->part, ev->npad);
   };
   if (ev->p.using_shear) {
     if (ev->no_bulk) go(k_grad_slice<true, false>); else go(k_grad_slice<true, true>);

@@ -113,24 +113,23 @@ struct Seg3 {
   double mn[3], mx[3];
 };
 
-// The (y, eta) cell-row segments of the tile owned by this wave.
+// The (y, eta) cell-row segments of the tile owned by this wave (runs of
+// lanes: sorted positions have ascending key rows).
 template <class Fn>
 __device__ __forceinline__ void for_segments3(bool act, int myrow, const double* r, Fn&& fn)
 {
-  bool done = !act;
-  for (;;) {
-    const int row = uni(wave_min_i(done ? INT_MAX : myrow));
-    if (row == INT_MAX) break;
-    const bool in = !done && myrow == row;
+  uint64_t todo = __ballot(act);
+  while (todo) {
     Seg3 s;
-    s.row = row;
+    s.row = __builtin_amdgcn_readlane(myrow, __builtin_ctzll(todo));
+    const bool in = act && myrow == s.row;
     #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      s.mn[d] = uni(wave_min_d(in ? r[d] : INFINITY));
-      s.mx[d] = uni(wave_max_d(in ? r[d] : -INFINITY));
+      s.mn[d] = wave_min_d(in ? r[d] : INFINITY);
+      s.mx[d] = wave_max_d(in ? r[d] : -INFINITY);
     }
     fn(s, in);
-    done = done || in;
+    todo &= ~__ballot(in);
   }
 }
 
@@ -184,7 +183,7 @@ __device__ __forceinline__ void for_spans_slice3(const Grid& g, const int32_t* _
   for (int r0 = 0; r0 < nrow; r0 += kWave) {
     int b2, e2;
     row_run3(g, cell_off, s, rcs, ry0, nry, rz0, nrow, r0 + lane, b2, e2);
-    tot += uni(wave_sum_i(e2 - b2));
+    tot += last_lane(wave_incl_scan_i(e2 - b2));
   }
   const int lo = (int)(((long long)tot * slice) / nslices);
   const int hi = (int)(((long long)tot * (slice + 1)) / nslices);
@@ -193,8 +192,8 @@ __device__ __forceinline__ void for_spans_slice3(const Grid& g, const int32_t* _
     int b, e;
     row_run3(g, cell_off, s, rcs, ry0, nry, rz0, nrow, r0 + lane, b, e);
     const int len = e - b;
-    const int pre = wave_excl_scan_i(len);
-    const int ctot = uni(wave_sum_i(len));
+    const int incl = wave_incl_scan_i(len), pre = incl - len;
+    const int ctot = last_lane(incl);
     const int nr = nrow - r0 < kWave ? nrow - r0 : kWave;
     for (int r = 0; r < nr; ++r) {
       const int rbase = base + __builtin_amdgcn_readlane(pre, r);

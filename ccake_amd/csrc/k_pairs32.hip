@@ -71,6 +71,45 @@ __global__ __launch_bounds__(256) void k_records32(const double* __restrict__ ca
   else grad_record32(cand + (size_t)k * kCandG, out + (size_t)k * kCandG32);
 }
 
+// Slice `slice` of a segment's candidate runs, run by run (every lane active).
+template <class Body>
+__device__ __forceinline__ void for_runs_slice(const Grid& g, const int32_t* __restrict__ cell_off,
+                                                const Seg& s, double rcs, int slice, int nslices, Body&& body)
+{
+  const int lane = threadIdx.x & (kWave - 1);
+  const int ry0 = uni(cell_of(s.ymn - rcs, g.lo[1], g.inv_cell, g.nc[1]));
+  const int ry1 = uni(cell_of(s.ymx + rcs, g.lo[1], g.inv_cell, g.nc[1]));
+  const int nrow = ry1 - ry0 + 1;
+  int b, e;
+  row_run(g, cell_off, s, rcs, ry0, nrow, lane, b, e);
+  int tot = last_lane(wave_incl_scan_i(e - b));
+  for (int r0 = kWave; r0 < nrow; r0 += kWave) {     // more than 64 rows: rare
+    int b2, e2;
+    row_run(g, cell_off, s, rcs, ry0, nrow, r0 + lane, b2, e2);
+    tot += last_lane(wave_incl_scan_i(e2 - b2));
+  }
+  const int lo = (int)(((long long)tot * slice) / nslices);
+  const int hi = (int)(((long long)tot * (slice + 1)) / nslices);
+  int base = 0;
+  for (int r0 = 0; r0 < nrow && base < hi; r0 += kWave) {
+    if (r0 > 0) row_run(g, cell_off, s, rcs, ry0, nrow, r0 + lane, b, e);
+    const int len = e - b;
+    const int incl = wave_incl_scan_i(len), pre = incl - len;
+    const int ctot = last_lane(incl);
+    const int nr = nrow - r0 < kWave ? nrow - r0 : kWave;
+    for (int r = 0; r < nr; ++r) {
+      const int rbase = base + __builtin_amdgcn_readlane(pre, r);
+      if (rbase >= hi) break;
+      const int rb = __builtin_amdgcn_readlane(b, r);
+      const int rlen = __builtin_amdgcn_readlane(len, r);
+      const int t0 = lo > rbase ? lo - rbase : 0;
+      const int t1 = hi - rbase < rlen ? hi - rbase : rlen;
+      if (t0 < t1) body(rb + t0, rb + t1);
+    }
+    base += ctot;
+  }
+}
+
 // walk_records over FP32 records: NR dwords of each record (wave-uniform
 // scalar loads), U records per step with the next U requested while the
 // current ones are evaluated (the same ordering as walk_records), and
@@ -114,6 +153,10 @@ __device__ __forceinline__ void walk_records32(const uint32_t* __restrict__ cand
   }
   fold();
 }
+
+// Where a lane outside the segment stands: its r^2 = 1e30 is finite in FP32,
+// so every candidate's weight is an exact 0 and so are its terms.
+constexpr double kFarAway32 = 1e15;
 
 // q = r/h and 1/q in FP32 from the FP64 r^2: v_rsq_f32 of q^2 (1e-30 added
 // so that coincident particles get q ~ 1e-15 and a zero gradient).
@@ -174,9 +217,10 @@ __global__ __launch_bounds__(kWave * (W > 0 ? W : 1)) void k_smooth_slice32(cons
 
   for_segments(act, myrow, xi, yi, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    for_spans_slice(g, cell_off, seg, rcs, slice, nslices, in, [&](int j0, int j1) {
+    const double xs = in ? xi : kFarAway32;    // lanes of other cell rows sit this segment's walk out
+    for_runs_slice(g, cell_off, seg, rcs, slice, nslices, [&](int j0, int j1) {
       constexpr int NR = (MODE == 0) ? 9 : 6;
-      walk_records32<NR, kCandS32, U, FOLD>(cand, xi, yi, j0, j1,
+      walk_records32<NR, kCandS32, U, FOLD>(cand, xs, yi, j0, j1,
                                       [&](const uint32_t* c, double dx, double dy, int j, bool valid) {
         const double r2 = dist2_nocontract(dx, dy);
         const bool nb = valid && r2 <= rc2;
@@ -264,9 +308,10 @@ void k_grad_slice32(const double* __restrict__ cand64,
 
   for_segments(act, myrow, xa, ya, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    for_spans_slice(g, cell_off, seg, rcs, slice, nslices, in, [&](int j0, int j1) {
+    const double xs = in ? xa : kFarAway32;    // lanes of other cell rows sit this segment's walk out
+    for_runs_slice(g, cell_off, seg, rcs, slice, nslices, [&](int j0, int j1) {
       constexpr int NR = SHEAR ? 15 : 10;
-      walk_records32<NR, kCandG32, 2, FOLD>(cand, xa, ya, j0, j1,
+      walk_records32<NR, kCandG32, 2, FOLD>(cand, xs, ya, j0, j1,
                                       [&](const uint32_t* c, double dx, double dy, int j, bool valid) {
         const double r2 = dist2_nocontract(dx, dy);
         if (kSkipEmpty && wave_none(valid && r2 <= rc2)) return;

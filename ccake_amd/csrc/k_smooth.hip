@@ -152,14 +152,18 @@ template <int MODE>
 constexpr int smooth_nacc() { return (MODE == 0 || MODE == 3) ? 6 : 2; }
 
 // The walk of one (tile, slice) unit (one wave); fin(acc) receives the
-// slice's sums (sigma_lab, the pair count, then s, B, S, Q).
-template <int MODE, class Fin>
+// slice's sums (sigma_lab, the pair count, then s, B, S, Q).  KEEP: with the
+// arithmetic of q_and_inverse and spline_w (keep_order).
+// Bound: the FP64 vector unit, 23 instructions per candidate and wave in
+// MODE 0.  188,250 particles (479M pairs): 745 us per launch with 31
+// instructions and no request ahead, 610 us now.
+template <int MODE, bool KEEP, class Fin>
 __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, const int32_t* __restrict__ skey,
                                             const int32_t* __restrict__ cell_off, const Grid* __restrict__ gridp,
-                                            int n, double rc2, double rcs, double hinv2, int tile, int slice,
+                                            int n, double rc2, double rcs, double hinv2, double m4h, double mk2h, int tile, int slice,
                                             int nslices, Fin&& fin)
 {
-  const Grid g0 = *gridp;
+  const Grid& g0 = *gridp;
   const int lane = threadIdx.x & (kWave - 1);
   const int k = tile * kTile + lane;
   const bool act = k < n;
@@ -173,19 +177,21 @@ __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, con
 
   for_segments(act, myrow, xi, yi, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    // lanes of other cell rows sit this segment's walk out
-    for_spans_slice(g, cell_off, seg, rcs, slice, nslices, in, [&](int j0, int j1) {
-      // wave-uniform candidate records (scalar loads into SGPRs)
-      constexpr int NR = (MODE == 0) ? 7 : (MODE == 3 ? 4 : 3);
-      walk_records<NR, kCandS, 2>(cand, xi, yi, j0, j1,
-                                  [&](const double* c, double dx, double dy, int j, bool valid) {
-        const double r2 = dist2_nocontract(dx, dy);
-        const bool nb = valid && r2 <= rc2;
-        cnt += nb ? 1 : 0;
-        if (kSkipEmpty && wave_none(nb)) return;
-        double q, iq;
-        q_and_inverse(r2, hinv2, q, iq);
-        const double w = valid ? spline_w(q) : 0.0;
+    const double xs = in ? xi : kFarAway;      // lanes of other cell rows sit this segment's walk out
+    for_spans_slice<kCandS, KEEP>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
+      // whole records or half records: one scalar load each
+      constexpr int NR = (MODE == 0) ? 8 : 4;
+      walk_records<NR, kCandS, 1>(cand, xs, yi, cur,
+                               [&](const double* c, double dx, double dy, double r2) {
+        cnt += r2 <= rc2 ? 1 : 0;
+        double w;
+        if (KEEP) {
+          double q, iq;
+          q_and_inverse(r2, hinv2, q, iq);
+          w = spline_w(q);
+        } else {
+          w = spline_w8(r2, m4h, mk2h);
+        }
         sl += c[2] * w;
         if (MODE == 0 || MODE == 3) ss += c[MODE == 1 ? 0 : 3] * w;
         if (MODE == 0) {
@@ -195,7 +201,8 @@ __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, con
       });
     });
   });
-  const double acc[6] = { sl, (double)cnt, ss, sB, sS, sQ };
+  const double f = KEEP ? 1.0 : kSplineW;
+  const double acc[6] = { f * sl, (double)cnt, f * ss, f * sB, f * sS, f * sQ };
   fin(acc);
 }
 
@@ -204,14 +211,14 @@ __global__ __launch_bounds__(kWave) void k_smooth_slice(const double* __restrict
                                                         const int32_t* __restrict__ skey,
                                                         const int32_t* __restrict__ cell_off,
                                                         const Grid* __restrict__ gridp, int n,
-                                                        double rc2, double rcs, double hinv2, int nslices,
+                                                        double rc2, double rcs, double hinv2, double m4h, double mk2h, int nslices,
                                                         double* __restrict__ part, int npad)
 {
   constexpr int NACC = smooth_nacc<MODE>();
   const int unit = xcd_tile(blockIdx.x, gridDim.x);
   const int tile = unit / nslices;
   const int slice = unit - tile * nslices;
-  smooth_walk<MODE>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, tile, slice, nslices, [&](const double* acc) {
+  smooth_walk<MODE, false>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, mk2h, tile, slice, nslices, [&](const double* acc) {
     double* p = part + (size_t)slice * NACC * npad + tile * kTile + threadIdx.x;
     #pragma unroll
     for (int q = 0; q < NACC; ++q) p[(size_t)q * npad] = acc[q];
@@ -220,12 +227,12 @@ __global__ __launch_bounds__(kWave) void k_smooth_slice(const double* __restrict
 
 // The W slices of a tile in one workgroup of W waves, their sums added in
 // slice order in LDS and stored as one slice's (as k_grad_tile).
-template <int MODE, int W>
+template <int MODE, int W, bool KEEP = false>
 __global__ __launch_bounds__(kWave * W) void k_smooth_tile(const double* __restrict__ cand,
                                                            const int32_t* __restrict__ skey,
                                                            const int32_t* __restrict__ cell_off,
                                                            const Grid* __restrict__ gridp, int n,
-                                                           double rc2, double rcs, double hinv2,
+                                                           double rc2, double rcs, double hinv2, double m4h, double mk2h,
                                                            double* __restrict__ part, int npad)
 {
   constexpr int NACC = smooth_nacc<MODE>();
@@ -233,7 +240,7 @@ __global__ __launch_bounds__(kWave * W) void k_smooth_tile(const double* __restr
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int slice = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // wave-uniform
   const int lane = threadIdx.x & (kWave - 1);
-  smooth_walk<MODE>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, tile, slice, W, [&](const double* acc) {
+  smooth_walk<MODE, KEEP>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, mk2h, tile, slice, W, [&](const double* acc) {
     #pragma unroll
     for (int q = 0; q < NACC; ++q) red[slice][q][lane] = acc[q];
   });
@@ -347,17 +354,22 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
   }
   if (mode == 0 && ev->p.pair_precision == 1) return launch_smooth_pairs32(ev);
-  const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT);
+  const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT), m4h = -0.25 / ev->p.hT, mk2h = -0.5 * kSplineK / ev->p.hT;
   const int W = lds_slices(ev);
   if (W) {
     // the tile's slices reduced in LDS: the sum pass sees one slice
     ev->smooth_sum_slices = 1;
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kWave * W), 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n,
-                         rc2, rcs, hinv2, ev->part, ev->npad);
+    auto launch = [&](auto kern, int waves) {
+      hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kWave * waves), 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n,
+                         rc2, rcs, hinv2, m4h, mk2h, ev->part, ev->npad);
     };
+    auto go = [&](auto kern) { launch(kern, W); };
     const int m = (mode == 0 && ev->no_charges) ? 3 : mode;
-    if (W == 8) { if (m == 3) go(k_smooth_tile<3, 8>); else if (m == 0) go(k_smooth_tile<0, 8>); else go(k_smooth_tile<1, 8>); }
+    if (W >= kKeepSmoothWaves && keep_order(ev, ntiles)) {
+      if (m == 3) launch(k_smooth_tile<3, kKeepSmoothWaves, true>, kKeepSmoothWaves);
+      else if (m == 0) launch(k_smooth_tile<0, kKeepSmoothWaves, true>, kKeepSmoothWaves);
+      else launch(k_smooth_tile<1, kKeepSmoothWaves, true>, kKeepSmoothWaves);
+    } else if (W == 8) { if (m == 3) go(k_smooth_tile<3, 8>); else if (m == 0) go(k_smooth_tile<0, 8>); else go(k_smooth_tile<1, 8>); }
     else { if (m == 3) go(k_smooth_tile<3, 4>); else if (m == 0) go(k_smooth_tile<0, 4>); else go(k_smooth_tile<1, 4>); }
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
   }
@@ -365,13 +377,13 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
   const dim3 grid(ntiles * ev->nslices), blk(kWave);
   if (mode == 0 && ev->no_charges)
     hipLaunchKernelGGL(k_smooth_slice<3>, grid, blk, 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n, rc2,
-                       rcs, hinv2, ev->nslices, ev->part, ev->npad);
+                       rcs, hinv2, m4h, mk2h, ev->nslices, ev->part, ev->npad);
   else if (mode == 0)
     hipLaunchKernelGGL(k_smooth_slice<0>, grid, blk, 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n, rc2,
-                       rcs, hinv2, ev->nslices, ev->part, ev->npad);
+                       rcs, hinv2, m4h, mk2h, ev->nslices, ev->part, ev->npad);
   else
     hipLaunchKernelGGL(k_smooth_slice<1>, grid, blk, 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n, rc2,
-                       rcs, hinv2, ev->nslices, ev->part, ev->npad);
+                       rcs, hinv2, m4h, mk2h, ev->nslices, ev->part, ev->npad);
   return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
 }
 

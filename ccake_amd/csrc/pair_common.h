@@ -11,20 +11,70 @@
 
 namespace ccake {
 
-__device__ __forceinline__ int wave_min_i(int v)
+// Wave reductions and scans over data-parallel moves (row shifts by 1, 2, 4
+// and 8 lanes, then the last lane of a row of 16 to the next row and of the
+// lower half to the upper): six dependent steps of a few cycles each, where
+// a shuffle through LDS takes over a hundred.  The setup of a pair walk is a
+// chain of them, which is most of a small event's pass.  Lane 63 ends with
+// the whole wave's result.  The host emulation build uses the shuffles.
+#ifndef CCAKE_HOST_EMU
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_move(int ident, int v)
 {
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
+  return __builtin_amdgcn_update_dpp(ident, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double ident, double v)
+{
+  const long long i = __double_as_longlong(ident), b = __double_as_longlong(v);
+  const int lo = dpp_move<CTRL, ROWS>((int)i, (int)b), hi = dpp_move<CTRL, ROWS>((int)(i >> 32), (int)(b >> 32));
+  return __hiloint2double(hi, lo);
+}
+// inclusive scan of `op` with identity `ident`
+template <class T, class Op>
+__device__ __forceinline__ T wave_scan(T v, T ident, Op&& op)
+{
+  v = op(v, dpp_move<0x111, 0xf>(ident, v));   // row_shr:1
+  v = op(v, dpp_move<0x112, 0xf>(ident, v));
+  v = op(v, dpp_move<0x114, 0xf>(ident, v));
+  v = op(v, dpp_move<0x118, 0xf>(ident, v));
+  v = op(v, dpp_move<0x142, 0xa>(ident, v));   // row_bcast:15 into rows 1 and 3
+  v = op(v, dpp_move<0x143, 0xc>(ident, v));   // row_bcast:31 into rows 2 and 3
   return v;
 }
+__device__ __forceinline__ int last_lane(int v) { return __builtin_amdgcn_readlane(v, kWave - 1); }
+__device__ __forceinline__ double last_lane(double v)
+{
+  const long long b = __double_as_longlong(v);
+  return __hiloint2double(__builtin_amdgcn_readlane((int)(b >> 32), kWave - 1),
+                          __builtin_amdgcn_readlane((int)b, kWave - 1));
+}
+#else
+template <class T, class Op>
+__device__ __forceinline__ T wave_scan(T v, T ident, Op&& op)
+{
+  const int lane = threadIdx.x & (kWave - 1);
+  for (int o = 1; o < kWave; o <<= 1) {
+    const T y = __shfl_up(v, o);
+    if (lane >= o) v = op(v, y);
+  }
+  return v;
+}
+template <class T>
+__device__ __forceinline__ T last_lane(T v) { return __shfl(v, kWave - 1); }
+#endif
+// wave-uniform results
 __device__ __forceinline__ double wave_min_d(double v)
 {
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
-  return v;
+  return last_lane(wave_scan(v, (double)INFINITY, [](double a, double b) { return fmin(a, b); }));
 }
 __device__ __forceinline__ double wave_max_d(double v)
 {
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
-  return v;
+  return last_lane(wave_scan(v, -(double)INFINITY, [](double a, double b) { return fmax(a, b); }));
+}
+__device__ __forceinline__ int wave_incl_scan_i(int v)
+{
+  return wave_scan(v, 0, [](int a, int b) { return a + b; });
 }
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ double uni(double v)
@@ -114,22 +164,6 @@ __device__ __forceinline__ int xcd_tile(int bid, int nblk)
 // even when there are few tiles.  Every wave of a tile computes the same
 // segments and spans (wave-uniform values).
 
-__device__ __forceinline__ int wave_sum_i(int v)
-{
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-__device__ __forceinline__ int wave_excl_scan_i(int v)
-{
-  const int lane = threadIdx.x & (kWave - 1);
-  int x = v;
-  for (int o = 1; o < kWave; o <<= 1) {
-    const int y = __shfl_up(x, o);
-    if (lane >= o) x += y;
-  }
-  return x - v;
-}
-
 // Candidate run of cell row ry0 + r for a segment: [b, e) in sorted order
 // (empty when r >= nrow or the row is out of reach).  Evaluated per lane.
 __device__ __forceinline__ void row_run(const Grid& g, const int32_t* __restrict__ cell_off, const Seg& s,
@@ -149,13 +183,6 @@ __device__ __forceinline__ void row_run(const Grid& g, const int32_t* __restrict
   e = cell_off[kr + cx1 + 1];
 }
 
-// Walk slice `slice` of `nslices` of a segment's flattened candidate list
-// (rows ascending, cells ascending within a row).  The rows are resolved
-// lane-parallel, lane r holding cell row ry0 + r (64 rows at a time), so
-// the cell offsets of every row arrive with one vector load; the walk reads
-// a row's run back with readlane.  Called with every lane of the wave
-// active; body(j0, j1) runs on the lanes with `in` set, with wave-uniform
-// sorted indices j0 < j1.
 // Skip a candidate (wave-uniform branch) when it is out of range for every
 // active lane: such candidates lie in the cell-rounding margin of the
 // tile's region, and every lane would add exact zeros.  On by default
@@ -181,10 +208,82 @@ __device__ __forceinline__ bool wave_none(bool p)
 #endif
 }
 
-template <class Body>
+// The candidates of one slice of a segment that can be in range, in order,
+// 64 cell rows' worth (the rows are resolved lane-parallel, lane r holding
+// row r's run, so their cell offsets arrive with one vector load).  The
+// slice's flattened list is taken in batches of 64, a candidate per lane:
+// the lanes find their candidates' sorted indices, load their positions and
+// keep those no farther than the cutoff from the segment's bounding box.  At
+// the ends of the runs, which follow the cutoff disc only to a cell row, that
+// drops one candidate in five (188,250 particles) at a 64th of the cost of
+// meeting it in the walk, where it would still wait for its record.  The
+// positions of a batch are requested before the one in hand is walked; they
+// also bring the records' lines into the L2, which the walk's scalar loads
+// would go past one by one.
+struct RunCursor {
+  // lane r: the flattened index of row r's first candidate, its sorted index, the run's length
+  int first, run, len;
+  int t, hi, step;                // wave-uniform: flattened index of the next batch's first candidate, the slice's
+                                  // end, and how far apart its candidates are (1, or the number of slices)
+  const double* pos;              // records with x, y in front
+  int stride;
+  const Seg* seg;
+  double far2;                    // square of the cutoff with a margin for rounding
+  uint64_t mask = 0;              // lanes of the batch in hand that are still to visit
+  int j = 0;                      // their sorted indices
+  bool ahead = false;             // a batch is requested: jn, vn, xn, yn
+  int jn = 0;
+  bool vn = false;
+  double xn = 0.0, yn = 0.0;
+
+  __device__ __forceinline__ void request()
+  {
+    ahead = t < hi;
+    if (!ahead) return;
+    const int q = t + step * (int)(threadIdx.x & (kWave - 1));
+    vn = q < hi;
+    jn = 0;
+    for (uint64_t m = __ballot(len > 0 && first < t + kWave * step && first + len > t); m; m &= m - 1) {
+      const int r = __builtin_ctzll(m);
+      const int f = __builtin_amdgcn_readlane(first, r), l = __builtin_amdgcn_readlane(len, r);
+      const int s = __builtin_amdgcn_readlane(run, r);
+      if (q >= f && q < f + l) jn = s + q - f;
+    }
+    xn = pos[(size_t)jn * stride];
+    yn = pos[(size_t)jn * stride + 1];
+    t += kWave * step;
+  }
+  // the next candidate's sorted index (wave-uniform), -1 after the last
+  __device__ __forceinline__ int next()
+  {
+    while (mask == 0) {
+      if (!ahead) return -1;
+      const double bx = fmax(fmax(seg->xmn - xn, xn - seg->xmx), 0.0);
+      const double by = fmax(fmax(seg->ymn - yn, yn - seg->ymx), 0.0);
+      mask = __ballot(vn && bx * bx + by * by <= far2);
+      j = jn;
+      request();
+    }
+    const int l = __builtin_ctzll(mask);
+    mask &= mask - 1;
+    return __builtin_amdgcn_readlane(j, l);
+  }
+};
+
+// Slice `slice` of `nslices` of a segment's flattened candidate list (rows
+// ascending, cells ascending within a row): every nslices-th candidate, so
+// that the slices have equal shares of every row.  (Contiguous slices have
+// equal shares of the list, but the first and the last have more of it out of
+// range, and they are always the same SIMDs' waves: gradients of
+// 188,250 particles 987 us contiguous, 965 dealt out.)
+// KEEP: contiguous all the same (keep_order).  body(cursor) once per 64 cell
+// rows that hold some of the slice.  Called with every lane of the wave
+// active; body runs on every lane (wave-uniform control flow): a lane outside
+// the segment stands at kFarAway, which every candidate's weight is 0 for.
+template <int STRIDE, bool KEEP, class Body>
 __device__ __forceinline__ void for_spans_slice(const Grid& g, const int32_t* __restrict__ cell_off,
-                                                const Seg& s, double rcs, int slice, int nslices, bool in,
-                                                Body&& body)
+                                                const double* __restrict__ cand, const Seg& s, double rc2, double rcs,
+                                                int slice, int nslices, Body&& body)
 {
   const int lane = threadIdx.x & (kWave - 1);
   const int ry0 = uni(cell_of(s.ymn - rcs, g.lo[1], g.inv_cell, g.nc[1]));
@@ -192,31 +291,39 @@ __device__ __forceinline__ void for_spans_slice(const Grid& g, const int32_t* __
   const int nrow = ry1 - ry0 + 1;
   int b, e;
   row_run(g, cell_off, s, rcs, ry0, nrow, lane, b, e);
-  int tot = uni(wave_sum_i(e - b));
-  for (int r0 = kWave; r0 < nrow; r0 += kWave) {     // more than 64 rows: rare
-    int b2, e2;
-    row_run(g, cell_off, s, rcs, ry0, nrow, r0 + lane, b2, e2);
-    tot += uni(wave_sum_i(e2 - b2));
+  int incl = wave_incl_scan_i(e - b);
+  int tot = last_lane(incl);
+  int lo = 0, hi = INT_MAX;
+  if (KEEP) {
+    for (int r0 = kWave; r0 < nrow; r0 += kWave) {     // more than 64 rows: rare
+      int b2, e2;
+      row_run(g, cell_off, s, rcs, ry0, nrow, r0 + lane, b2, e2);
+      tot += last_lane(wave_incl_scan_i(e2 - b2));
+    }
+    lo = (int)(((long long)tot * slice) / nslices);
+    hi = (int)(((long long)tot * (slice + 1)) / nslices);
   }
-  const int lo = (int)(((long long)tot * slice) / nslices);
-  const int hi = (int)(((long long)tot * (slice + 1)) / nslices);
   int base = 0;
   for (int r0 = 0; r0 < nrow && base < hi; r0 += kWave) {
-    if (r0 > 0) row_run(g, cell_off, s, rcs, ry0, nrow, r0 + lane, b, e);
-    const int len = e - b;
-    const int pre = wave_excl_scan_i(len);
-    const int ctot = uni(wave_sum_i(len));
-    const int nr = nrow - r0 < kWave ? nrow - r0 : kWave;
-    for (int r = 0; r < nr; ++r) {
-      const int rbase = base + __builtin_amdgcn_readlane(pre, r);
-      if (rbase >= hi) break;
-      const int rb = __builtin_amdgcn_readlane(b, r);
-      const int rlen = __builtin_amdgcn_readlane(len, r);
-      const int t0 = lo > rbase ? lo - rbase : 0;
-      const int t1 = hi - rbase < rlen ? hi - rbase : rlen;
-      if (t0 < t1 && in) body(rb + t0, rb + t1);
+    if (r0 > 0) {
+      row_run(g, cell_off, s, rcs, ry0, nrow, r0 + lane, b, e);
+      incl = wave_incl_scan_i(e - b);
     }
-    base += ctot;
+    const int end = base + last_lane(incl);
+    RunCursor c;
+    c.run = b;
+    c.len = e - b;
+    c.first = base + incl - c.len;
+    c.t = KEEP ? (lo > base ? lo : base) : base + slice;
+    c.hi = hi < end ? hi : end;
+    c.step = KEEP ? 1 : nslices;
+    c.pos = cand;
+    c.stride = STRIDE;
+    c.seg = &s;
+    c.far2 = rc2 * (1.0 + 1e-9);
+    c.request();
+    body(c);
+    base = end;
   }
 }
 
@@ -236,52 +343,124 @@ inline int choose_slices(int ntiles, int simds)
   return best;
 }
 
+// Slices per tile of the 2+1D kernels, which run a tile's slices as the waves
+// of one workgroup.  More do not pay even where 8 leave SIMDs empty (2,601
+// particles, 41 tiles: smoothing and gradients 55 us a stage with 8, 58 with
+// 16), and 16 cost where they do not (30,300 particles: 128 against 142 us).
+constexpr int kTileWaves = 8;
+// The gradient walk's waves are longer: 4 once they fill the SIMDs (188,250
+// particles, 2,942 tiles: 965 us with 4, 974 with 8; 182,355 in six events:
+// 349 against 369; 40,401 particles, 632 tiles: 96 us with 4, 89 with 8).
+inline int grad_tile_waves(int waves, int ntiles, int simds) { return waves == 8 && ntiles >= simds ? 4 : waves; }
+
+// A small event whose freeze-out hypersurface is recorded keeps one order and
+// one form of its pair sums: the hypersurface's divE column is the
+// reciprocal of a difference, so another rounding of the sums moves its worst
+// entries by 1e-11 to 2e-9 after the 300 steps to freeze-out (10 events of
+// 5,000 to 7,650 particles), and runs of it are compared entry by entry.
+// While the waves do not fill the chip a pass is the latency of its setup and
+// loads, and the shorter arithmetic gains little: smoothing and gradients of
+// 7,650 particles take 31 and 51 us in this form, 30 and 40 in the other with
+// 8 waves per tile.
+inline bool keep_order(const ccake_event* ev, int ntiles)
+{
+  return ev->snaps && 8 * ntiles <= ev->dev->simds;
+}
+constexpr int kKeepSmoothWaves = 8, kKeepGradWaves = 4;
+
 // Per-slice partial sums: part[(slice * nacc + f) * npad + k] for sorted
 // position k (every tile lane, k < ntiles * 64 <= npad, has a slot).
 constexpr int kMaxAcc = 17;
 constexpr int kMaxSlices = 16;
 
-// Walk candidates j0 .. j1-1 (wave-uniform) U at a time with the next U
-// records requested while the current ones are evaluated.  Scalar loads may
-// return out of order, so a wait always covers every load in flight; the
-// first use of the current records (their offsets dx, dy) is therefore
-// pinned before the next request, and the wait for the next records falls
-// after the current arithmetic.  Indices past j1 - 1 are clamped (those
-// loads are in bounds and their results unused).  body(c, dx, dy, j, valid)
-// evaluates one candidate; `valid` is false for the padding slot of a short
-// last step.
+// Hold values at this point of the program: what uses them is not scheduled
+// above it, and the loads that made them are not sunk below it.
+__device__ __forceinline__ void pin_vector(double& a, double& b)
+{
+#ifndef CCAKE_HOST_EMU
+  asm volatile("" : "+v"(a), "+v"(b));
+#endif
+}
+template <int NR>
+__device__ __forceinline__ void pin_scalar(const double (&r)[NR])
+{
+#ifndef CCAKE_HOST_EMU
+  __builtin_amdgcn_sched_barrier(0);
+  #pragma unroll
+  for (int q = 0; q < NR; ++q) asm volatile("" :: "s"(r[q]));
+#endif
+}
+
+// One step of walk_records: the U records of `cur` are evaluated (the first
+// alone when there is no second) while those at sorted indices n[] are
+// requested.  A wait on scalar loads covers every one in flight (they can
+// return out of order), so the wait for `cur` is taken by its offsets, before
+// the request (pin_vector), and the wait for `nxt` falls after the whole of
+// this step's arithmetic (pin_scalar: the compiler would otherwise move its
+// loads to their use in the next step).
 template <int NR, int STRIDE, int U, class Body>
-__device__ __forceinline__ void walk_records(const double* __restrict__ cand, double xi, double yi, int j0, int j1,
+__device__ __forceinline__ void walk_step(const double (&cur)[U][NR], double (&nxt)[U][NR],
+                                          const double* __restrict__ cand, const int (&n)[U], bool whole, double xi,
+                                          double yi, Body&& body)
+{
+  double dx[U], dy[U];
+  #pragma unroll
+  for (int u = 0; u < U; ++u) {
+    dx[u] = xi - cur[u][0];
+    dy[u] = yi - cur[u][1];
+    pin_vector(dx[u], dy[u]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  #pragma unroll
+  for (int u = 0; u < U; ++u)
+    #pragma unroll
+    for (int q = 0; q < NR; ++q) nxt[u][q] = cand[(size_t)n[u] * STRIDE + q];
+  __builtin_amdgcn_sched_barrier(0);
+  #pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (u == 0 || whole) body(cur[u], dx[u], dy[u], dist2_nocontract(dx[u], dy[u]));
+  #pragma unroll
+  for (int u = 0; u < U; ++u) pin_scalar<NR>(nxt[u]);
+}
+
+// Walk the candidates of a cursor, their records in scalar registers, U at a
+// time (1 or 2) and the next U requested ahead into the other of two register
+// sets: with one set and a copy, the loads of a record cannot be issued
+// before the last use of the one it replaces, and every candidate waits for
+// its own loads.  body(c, dx, dy, r2) adds one candidate's terms.
+template <int NR, int STRIDE, int U, class Body>
+__device__ __forceinline__ void walk_records(const double* __restrict__ cand, double xi, double yi, RunCursor& cur,
                                              Body&& body)
 {
   static_assert(U == 1 || U == 2, "one or two records per step");
-  if (j0 >= j1) return;
-  double cur[U][NR];
-  #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int ju = j0 + u < j1 ? j0 + u : j1 - 1;
-    #pragma unroll
-    for (int q = 0; q < NR; ++q) cur[u][q] = cand[(size_t)ju * STRIDE + q];
-  }
-  for (int j = j0; j < j1; j += U) {
-    double dx[U], dy[U];
-    #pragma unroll
-    for (int u = 0; u < U; ++u) { dx[u] = xi - cur[u][0]; dy[u] = yi - cur[u][1]; }
-    __builtin_amdgcn_sched_barrier(0);
-    double nxt[U][NR];
-    #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int ju = j + U + u < j1 ? j + U + u : j1 - 1;
-      #pragma unroll
-      for (int q = 0; q < NR; ++q) nxt[u][q] = cand[(size_t)ju * STRIDE + q];
+  double a[U][NR], b[U][NR];
+  int n[U];                       // the next records' indices; a missing one repeats the one before (in bounds, unused)
+  int count;                      // how many of them there are
+  auto take = [&]() {
+    const int j = cur.next();
+    count = j < 0 ? 0 : 1;
+    if (j >= 0) n[0] = j;
+    if (U == 2) {
+      const int k = j < 0 ? -1 : cur.next();
+      count += k < 0 ? 0 : 1;
+      n[U - 1] = k < 0 ? n[0] : k;
     }
-    __builtin_amdgcn_sched_barrier(0);
+  };
+  take();
+  if (count == 0) return;
+  #pragma unroll
+  for (int u = 0; u < U; ++u)
     #pragma unroll
-    for (int u = 0; u < U; ++u) body(cur[u], dx[u], dy[u], j + u, j + u < j1);
-    #pragma unroll
-    for (int u = 0; u < U; ++u)
-      #pragma unroll
-      for (int q = 0; q < NR; ++q) cur[u][q] = nxt[u][q];
+    for (int q = 0; q < NR; ++q) a[u][q] = cand[(size_t)n[u] * STRIDE + q];
+  for (;;) {
+    bool whole = count == U;
+    take();
+    walk_step<NR, STRIDE, U>(a, b, cand, n, whole, xi, yi, body);
+    if (count == 0) break;
+    whole = count == U;
+    take();
+    walk_step<NR, STRIDE, U>(b, a, cand, n, whole, xi, yi, body);
+    if (count == 0) break;
   }
 }
 
@@ -321,24 +500,65 @@ __device__ __forceinline__ double spline_g(double q, double iq)
   return fma(-4.0, u * u, t * t) * iq;
 }
 
+// The same kernel arithmetic in fewer instructions, from r^2 and 1/h:
+//   x = r^2 + 1e-300, y = v_rsq_f64(x), f = x y, e = 3 - f y (2 to the
+//   instruction's error): f e = 2 r and y e = 2 / r
+// is the Newton step of q_and_inverse without its two halvings, and with
+//   t = clamp(1 - r / 2h), u = clamp(1 - r / h)   (to [0, 1], one instruction each)
+// spline_g(q, 1/q) = 2 h (t^2 - u^2) (2 / r) and
+// spline_w(q) = 8 (t^3 - (k u)^3), k = 2^(-1/3): the clamps make the cut at
+// 2h and the switch at h.  The walks apply the factors 2 h and 8 once per
+// particle.  A lane whose position is kFarAway gets exactly 0 from every
+// candidate (r^2 = 1e200 stays finite).
+constexpr double kFarAway = 1e100;
+constexpr double kSplineW = 8.0;                     // spline_w / spline_w8
+__device__ __forceinline__ double clamp01(double v) { return fmin(fmax(v, 0.0), 1.0); }
+// 2 r of a pair; ir2 receives 2 / r
+__device__ __forceinline__ double twice_r(double r2, double& ir2)
+{
+  const double x = r2 + 1e-300;
+  const double y = __builtin_amdgcn_rsq(x);
+  const double f = x * y;
+  const double e = fma(-f, y, 3.0);
+  ir2 = y * e;
+  return f * e;
+}
+// (t^2 - u^2) * 2 / r; m4h = -1 / (4 h), m2h = -1 / (2 h)
+__device__ __forceinline__ double spline_g2(double r2, double m4h, double m2h)
+{
+  double ir2;
+  const double d = twice_r(r2, ir2);
+  const double t = clamp01(fma(d, m4h, 1.0)), u = clamp01(fma(d, m2h, 1.0));
+  return fma(-u, u, t * t) * ir2;
+}
+// t^3 - (k u)^3
+constexpr double kSplineK = 0.79370052598409973738;  // 2^(-1/3)
+__device__ __forceinline__ double spline_w8(double r2, double m4h, double mk2h)
+{
+  double ir2;
+  const double d = twice_r(r2, ir2);
+  const double t = clamp01(fma(d, m4h, 1.0)), u = clamp01(fma(d, mk2h, kSplineK));
+  return fma(-(u * u), u, (t * t) * t);
+}
+
 // Iterate over the row segments of the tile owned by this wave.  `fn(seg,
 // in_seg)` runs once per segment with in_seg true on the lanes of the segment.
+// Sorted positions have ascending key rows, so a segment is a run of lanes.
 template <class Fn>
 __device__ __forceinline__ void for_segments(bool act, int myrow, double xi, double yi, Fn&& fn)
 {
-  bool done = !act;
-  for (;;) {
-    const int r = uni(wave_min_i(done ? INT_MAX : myrow));
-    if (r == INT_MAX) break;
-    const bool in = !done && myrow == r;
+  uint64_t todo = __ballot(act);
+  while (todo) {
+    const int r = __builtin_amdgcn_readlane(myrow, __builtin_ctzll(todo));
+    const bool in = act && myrow == r;
     Seg s;
     s.row = r;
-    s.xmn = uni(wave_min_d(in ? xi : INFINITY));
-    s.xmx = uni(wave_max_d(in ? xi : -INFINITY));
-    s.ymn = uni(wave_min_d(in ? yi : INFINITY));
-    s.ymx = uni(wave_max_d(in ? yi : -INFINITY));
+    s.xmn = wave_min_d(in ? xi : INFINITY);
+    s.xmx = wave_max_d(in ? xi : -INFINITY);
+    s.ymn = wave_min_d(in ? yi : INFINITY);
+    s.ymx = wave_max_d(in ? yi : -INFINITY);
     fn(s, in);
-    done = done || in;
+    todo &= ~__ballot(in);
   }
 }
 

@@ -1,0 +1,44 @@
+"""The pair walks at the edges of their tiles, batches and dispatch rules,
+against the oracle after initialization and one time step (1e-12, as the
+other parity tests: sums of at most a few thousand FP64 terms in another
+order)."""
+import numpy as np
+import pytest
+
+import ccake_amd  # noqa: F401
+from ccake_amd import config
+from parity_metrics import DERIVS, STATE
+from test_gpu_parity import Pair, compare, ints_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def cloud(n, half, seed=3):
+    """n jittered points with flow, charges and a smooth energy profile."""
+    rng = np.random.default_rng(seed)
+    m = int(np.ceil(np.sqrt(n)))
+    g = np.linspace(-half, half, m) if m > 1 else np.zeros(1)
+    x, y = (a.ravel()[:n] + rng.uniform(-0.01, 0.01, n) for a in np.meshgrid(g, g))
+    e = (5.0 + 20.0 * np.exp(-(x * x + y * y) / 8.0)) / config.HBARC_GEVFM
+    f = 0.02 * np.cos(x + 0.3 * y)
+    return dict(x=x, y=y, e=e, ux=0.1 * x / (half + 1), uy=-0.05 * y / (half + 1), rhoB=f * e, rhoS=0.5 * f * e,
+                rhoQ=-f * e)
+
+
+# one particle; a tile and its neighbours; the last size of the kept summation
+# order (8,192 with a hypersurface) and the first beyond it; 40 cells per
+# radius: more than 64 key rows within reach of a tile
+@pytest.mark.parametrize("n,half,cells,particlization,shear", [
+    (1, 0.5, 4, 0, 1), (63, 0.4, 4, 0, 1), (64, 0.4, 1, 1, 1), (65, 0.4, 4, 0, 0), (300, 0.5, 40, 0, 1),
+    (300, 0.5, 40, 1, 1), (8192, 4.5, 4, 1, 1), (8193, 4.5, 4, 1, 1), (8192, 4.5, 4, 0, 0)])
+def test_walk_edges(dev, orc, n, half, cells, particlization, shear):
+    eta = 0.08 if shear else 0.0
+    cfg = config.base_params(t0=0.6, dt=0.01, particlization=particlization, eta_mode=config.ETA_CONSTANT,
+                             constant_eta_over_s=eta, cells_per_rc=cells, x_subcells=4)
+    p = Pair(dev, orc, cfg, cloud(n, half))
+    p.initialize()
+    ints_equal(p.g, p.o, "BTRACK")
+    p.step(1)
+    ints_equal(p.g, p.o, "BTRACK")
+    compare(p.g, p.o, STATE + DERIVS, what=f"n={n} cells={cells} surface={particlization} shear={shear}")
+    p.close()
