@@ -527,6 +527,7 @@ int ccake_eos_create(ccake_dev* dev, const ccake_eos_desc* desc, ccake_eos** out
     nn *= (size_t)desc->dims[a];
     t.gmin[a] = desc->mins[a];
     t.gdel[a] = desc->dims[a] <= 1 ? 0.0 : (desc->maxs[a] - desc->mins[a]) / (desc->dims[a] - 1.0);
+    t.ginv[a] = (t.dims[a] <= 1 || std::fabs(t.gdel[a]) < 1e-30) ? 0.0 : 1.0 / t.gdel[a];
     t.mins[a] = desc->mins[a]; t.maxs[a] = desc->maxs[a];
   }
   e->h_tab = new double[nn * 17];

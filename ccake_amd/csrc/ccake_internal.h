@@ -77,6 +77,7 @@ struct EosMember {
   double mins[4], maxs[4];
   int dims[4];
   double gmin[4], gdel[4];
+  double ginv[4];           // 1 / gdel; 0 for an axis without extent
   // table: smallest and largest node value of (s, B, S, Q, e), the bounds of
   // the multilinear interpolant (dmin > dmax for members without them)
   double dmin[5], dmax[5];

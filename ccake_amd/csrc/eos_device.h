@@ -188,6 +188,50 @@ CK_HD bool table_cell(const EosMember& m, const double* x, int* ind, double* fr)
   return true;
 }
 
+// The weights of a table cell's corners along each axis: [axis][bit].
+CK_HD void corner_weights(const double* fr, double (&wa)[4][2])
+{
+  #pragma unroll
+  for (int a = 0; a < 4; ++a)
+    #pragma unroll
+    for (int b = 0; b < 2; ++b) wa[a][b] = fr[a] + b - 2.0 * b * fr[a];
+}
+// Node of a cell's first corner, and how many nodes further corner h is (the
+// same for every particle: scalar arithmetic).
+CK_HD size_t first_node(const EosMember& m, const int* ind)
+{
+  return (((size_t)ind[0] * m.dims[1] + ind[1]) * m.dims[2] + ind[2]) * m.dims[3] + ind[3];
+}
+CK_HD size_t corner_step(const EosMember& m, int h)
+{
+  const int b0 = (h >> 3) & 1, b1 = (h >> 2) & 1, b2 = (h >> 1) & 1, b3 = h & 1;
+  return (((size_t)b0 * m.dims[1] + b1) * m.dims[2] + b2) * m.dims[3] + b3;
+}
+CK_HD double corner_weight(const double (&wa)[4][2], int h)
+{
+  double w = 1.0;
+  w *= wa[0][(h >> 3) & 1];
+  w *= wa[1][(h >> 2) & 1];
+  w *= wa[2][(h >> 1) & 1];
+  w *= wa[3][h & 1];
+  return w;
+}
+// The table functions below request several corners' values before they use
+// the first of them (gathered() keeps the compiler from sinking the loads to
+// their uses): corner by corner, each waited for its own trip to memory, 16
+// in a row, which was most of the EoS stage (a density evaluation of a wave
+// 16.6 k cycles, the 4x4 solve beside it 1.7 k; 9.5 k now.  The stage's EoS
+// at 7,650 particles 106 -> 74 us, at 188,250 324 -> 250 us).
+CK_HD void gathered()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+  __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// Corners of a density evaluation in flight (8 and 16 measured alike).
+constexpr int kDensCorners = 8;
+
 // One table field at x: the same weights and the same accumulation order as
 // table_fields, so the value is the one table_fields gives; NaN outside.
 CK_HD double table_field_one(const EosMember& m, const double* tab, const double* x, int field)
@@ -195,22 +239,20 @@ CK_HD double table_field_one(const EosMember& m, const double* tab, const double
   int ind[4]; double fr[4];
   if (__builtin_isnan(x[0]) || __builtin_isnan(x[1]) || __builtin_isnan(x[2]) || __builtin_isnan(x[3]) || !table_cell(m, x, ind, fr))
     return NAN;
+  double wa[4][2], v[16];
+  corner_weights(fr, wa);
+  const double* c0 = tab + first_node(m, ind) * 17 + field;
+  #pragma unroll
+  for (int h = 0; h < 16; ++h) v[h] = c0[corner_step(m, h) * 17];
+  gathered();
   double r = 0.0;
-  for (int h = 0; h < 16; ++h) {
-    const int b0 = (h >> 3) & 1, b1 = (h >> 2) & 1, b2 = (h >> 1) & 1, b3 = h & 1;
-    double w = 1.0;
-    w *= fr[0] + b0 - 2.0 * b0 * fr[0];
-    w *= fr[1] + b1 - 2.0 * b1 * fr[1];
-    w *= fr[2] + b2 - 2.0 * b2 * fr[2];
-    w *= fr[3] + b3 - 2.0 * b3 * fr[3];
-    const size_t node = (((size_t)(ind[0] + b0) * m.dims[1] + (ind[1] + b1)) * m.dims[2] + (ind[2] + b2)) * m.dims[3]
-                        + (ind[3] + b3);
-    r += w * tab[node * 17 + field];
-  }
+  #pragma unroll
+  for (int h = 0; h < 16; ++h) r += corner_weight(wa, h) * v[h];
   return r;
 }
 
-// Table fields at x: all 17 (tab, stride 17) into r; NaN outside.
+// Table fields at x: all 17 (tab, stride 17) into r; NaN outside.  Four
+// corners' values (136 registers) are in flight at a time.
 CK_HD void table_fields(const EosMember& m, const double* tab, const double* x, double* r)
 {
   int ind[4]; double fr[4];
@@ -218,18 +260,27 @@ CK_HD void table_fields(const EosMember& m, const double* tab, const double* x, 
     for (int k = 0; k < 17; ++k) r[k] = NAN;
     return;
   }
+  double wa[4][2];
+  corner_weights(fr, wa);
+  const double* c0 = tab + first_node(m, ind) * 17;
+  #pragma unroll
   for (int k = 0; k < 17; ++k) r[k] = 0.0;
-  for (int h = 0; h < 16; ++h) {
-    const int b0 = (h >> 3) & 1, b1 = (h >> 2) & 1, b2 = (h >> 1) & 1, b3 = h & 1;
-    double w = 1.0;
-    w *= fr[0] + b0 - 2.0 * b0 * fr[0];
-    w *= fr[1] + b1 - 2.0 * b1 * fr[1];
-    w *= fr[2] + b2 - 2.0 * b2 * fr[2];
-    w *= fr[3] + b3 - 2.0 * b3 * fr[3];
-    const size_t node = (((size_t)(ind[0] + b0) * m.dims[1] + (ind[1] + b1)) * m.dims[2] + (ind[2] + b2)) * m.dims[3]
-                        + (ind[3] + b3);
-    const double* c = tab + node * 17;
-    for (int k = 0; k < 17; ++k) r[k] += w * c[k];
+  #pragma unroll
+  for (int g = 0; g < 16; g += 4) {
+    double v[4][17];
+    #pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const double* c = c0 + corner_step(m, g + h) * 17;
+      #pragma unroll
+      for (int k = 0; k < 17; ++k) v[h][k] = c[k];
+    }
+    gathered();
+    #pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const double w = corner_weight(wa, g + h);
+      #pragma unroll
+      for (int k = 0; k < 17; ++k) r[k] += w * v[h][k];
+    }
   }
 }
 
@@ -241,6 +292,16 @@ CK_HD void member_fields(const EosMember& m, const double* tab, const double* x,
   else if (has_kind<KM, M_TANH>() && m.kind == M_TANH) tanh_fields(m, x, r);
   else if (has_kind<KM, M_TABLE>()) table_fields(m, tab, x, r);
   else for (int k = 0; k < 17; ++k) r[k] = NAN;          // a kind outside the mask: never dispatched
+}
+
+// cs2 at x: the value member_fields gives, without the other 16 fields of a table.
+template <int KM = kAllMembers>
+CK_HD double member_cs2(const EosMember& m, const double* tab, const double* x)
+{
+  if (has_kind<KM, M_TABLE>() && m.kind == M_TABLE) return table_field_one(m, tab, x, X_CS2);
+  double r[17];
+  member_fields<KM & kAnalyticMembers>(m, nullptr, x, r);
+  return r[X_CS2];
 }
 
 // Residual densities (s|e, B, S, Q) at x and their Jacobian in (T, muB, muQ, muS).
@@ -256,25 +317,44 @@ CK_HD void member_dens(const EosMember& m, const double* tab5, int mode, const d
       for (int k = 0; k < 16; ++k) J[k] = NAN;
       return;
     }
+    #pragma unroll
     for (int k = 0; k < 4; ++k) F[k] = 0.0;
+    #pragma unroll
     for (int k = 0; k < 16; ++k) J[k] = 0.0;
-    double ga[4];
-    for (int a = 0; a < 4; ++a) ga[a] = (m.dims[a] <= 1 || fabs(m.gdel[a]) < 1e-30) ? 0.0 : 1.0 / m.gdel[a];
-    for (int h = 0; h < 16; ++h) {
-      const int bt[4] = { (h >> 3) & 1, (h >> 2) & 1, (h >> 1) & 1, h & 1 };
-      double wa[4];
-      double w = 1.0;
-      for (int a = 0; a < 4; ++a) { wa[a] = fr[a] + bt[a] - 2.0 * bt[a] * fr[a]; w *= wa[a]; }
-      const size_t node = (((size_t)(ind[0] + bt[0]) * m.dims[1] + (ind[1] + bt[1])) * m.dims[2] + (ind[2] + bt[2]))
-                          * m.dims[3] + (ind[3] + bt[3]);
-      const double* c = tab5 + node * 5;
-      const double v[4] = { mode ? c[4] : c[0], c[1], c[2], c[3] };
-      for (int k = 0; k < 4; ++k) F[k] += w * v[k];
+    double wa[4][2];
+    corner_weights(fr, wa);
+    const int f0 = mode ? 4 : 0;
+    const double* c0 = tab5 + first_node(m, ind) * 5;
+    #pragma unroll
+    for (int g = 0; g < 16; g += kDensCorners) {
+      double v[kDensCorners][4];
+      #pragma unroll
+      for (int h = 0; h < kDensCorners; ++h) {
+        const double* c = c0 + corner_step(m, g + h) * 5;
+        v[h][0] = c[f0];
+        #pragma unroll
+        for (int k = 1; k < 4; ++k) v[h][k] = c[k];
+      }
+      gathered();
+      #pragma unroll
+      for (int h = 0; h < kDensCorners; ++h) {
+        const double w = corner_weight(wa, g + h);
+        #pragma unroll
+        for (int k = 0; k < 4; ++k) F[k] += w * v[h][k];
+      }
+      // one branch per axis, not per corner and axis (each sum's corners stay in order)
+      #pragma unroll
       for (int a = 0; a < 4; ++a) {
-        if (ga[a] == 0.0) continue;
-        double dw = bt[a] ? ga[a] : -ga[a];
-        for (int b = 0; b < 4; ++b) if (b != a) dw *= wa[b];
-        for (int k = 0; k < 4; ++k) J[4 * k + a] += dw * v[k];
+        if (m.ginv[a] == 0.0) continue;
+        #pragma unroll
+        for (int h = 0; h < kDensCorners; ++h) {
+          const int bt[4] = { ((g + h) >> 3) & 1, ((g + h) >> 2) & 1, ((g + h) >> 1) & 1, (g + h) & 1 };
+          double dw = bt[a] ? m.ginv[a] : -m.ginv[a];
+          #pragma unroll
+          for (int b = 0; b < 4; ++b) if (b != a) dw *= wa[b][bt[b]];
+          #pragma unroll
+          for (int k = 0; k < 4; ++k) J[4 * k + a] += dw * v[h][k];
+        }
       }
     }
     return;
@@ -585,9 +665,8 @@ CK_HD int invert_first(const EosChain& ch, const double* tab, const double* tab5
   seed_of_kind(ch, mode, first_kind(mode), tgt, x, y0);
   root_seed(m, tgt, y0, 0, y);
   if (newton_attempt_b<KM>(m, tab5, mode, tgt, y, budget) != 1) return -1;
-  double r[17];
-  member_fields<KM>(m, tab, y, r);
-  if (r[X_CS2] < 0.0 || r[X_CS2] > 1.0) return -1;
+  const double cs2 = member_cs2<KM>(m, tab, y);
+  if (cs2 < 0.0 || cs2 > 1.0) return -1;
   for (int a = 0; a < 4; ++a) x[a] = y[a];
   *member = start;
   return 1;
@@ -628,9 +707,8 @@ __device__ bool invert_wave(const EosChain& ch, const double* tab, const double*
       const int first = __builtin_ctzll(mask);
       for (int a = 0; a < 4; ++a) res[a] = __shfl(y[a], first);
       used = k;
-      double r[17];
-      member_fields<KM>(m, tab, res, r);
-      if (r[X_CS2] < 0.0 || r[X_CS2] > 1.0) { for (int a = 0; a < 4; ++a) x[a] = res[a]; continue; }
+      const double cs2 = member_cs2<KM>(m, tab, res);
+      if (cs2 < 0.0 || cs2 > 1.0) { for (int a = 0; a < 4; ++a) x[a] = res[a]; continue; }
       break;
     }
   }
