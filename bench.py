@@ -567,7 +567,7 @@ def milne_run(dev, eos, steps=20, warmup=2):
                particle_steps_per_s=round(n * done / sec, 1), pairs_per_stage=int(pairs),
                neighbours_per_particle=round(pairs / n, 1),
                stage_ms={k: round(v[0] / max(v[1], 1), 4) for k, v in prof.items() if v[1]},
-               roofline=dict(kernel="k3_grad_slice", bound="valu", achieved=round(ach, 3), peak=PEAK_FP64_TFLOPS,
+               roofline=dict(kernel="k3_grad_tile", bound="valu", achieved=round(ach, 3), peak=PEAK_FP64_TFLOPS,
                              unit="TFLOP/s", frac=round(ach / PEAK_FP64_TFLOPS, 4),
                              work=f"{fg} flop/pair x {int(pairs)} pairs per launch", avg_launch_ms=round(gms, 4),
                              smoothing_frac=round(FLOP_PER_PAIR_SMOOTH3 * pairs / (sms * 1e-3) / 1e12

@@ -740,7 +740,7 @@ static int event_create(ccake_dev* dev, const ccake_params* p, ccake_eos* eos, i
   rc |= dalloc(ev, &ev->cell_off, (size_t)ev->cap_cells + 1);
   rc |= dalloc(ev, &ev->pair_count, 2);
   const int cap = choose_slices((n + kTile - 1) / kTile, dev->simds);
-  ev->nslices = p->dim == 3 ? cap : kTileWaves;
+  ev->nslices = p->dim == 3 ? kTileWaves3 : kTileWaves;
   if (const char* ov = std::getenv("CCAKE_PAIR_SLICES")) {     // tuning override, 1..16
     const int v = std::atoi(ov);
     if (v >= 1 && v <= kMaxSlices) ev->nslices = v;
@@ -752,8 +752,8 @@ static int event_create(ccake_dev* dev, const ccake_params* p, ccake_eos* eos, i
     if (v >= 0.0 && v <= 1.0) ev->skin_frac = v;
   }
   ev->nslices_cap = std::max(ev->nslices, cap);
-  // partial sums: 17 per slice in 2+1D, 28 in 3+1D (the 3D gradient sums)
-  rc |= dalloc(ev, &ev->part, (size_t)ev->nslices_cap * (p->dim == 3 ? 28 : kMaxAcc) * np);
+  // partial sums: 17 per slice in 2+1D, the smoothing sums in 3+1D
+  rc |= dalloc(ev, &ev->part, (p->dim == 3 ? (size_t)6 : (size_t)ev->nslices_cap * kMaxAcc) * np);
   rc |= dalloc(ev, &ev->hard, np);
   {
     // the EoS stage in two kernels (table chains): CCAKE_EOS_SPLIT=0 keeps one

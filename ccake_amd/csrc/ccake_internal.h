@@ -362,7 +362,7 @@ __device__ __forceinline__ void smooth_record(const double* __restrict__ F, int 
 // 3+1D candidate records.  Smoothing (8 doubles): x, y, eta, m_s,
 // m_s*ext_s, m_B*ext_B, m_S*ext_S, m_Q*ext_Q.  Gradients (24): x, y, eta,
 // m_s, p/sl^2, e, Pi/sl^2, v^x, v^y, v^eta, pi^{0i}/sl^2 (3), the spatial
-// pi^{ij}/sl^2 (xx, xy, x eta, yy, y eta, eta eta), sl, 4 unused.
+// pi^{ij}/sl^2 (xx, xy, x eta, yy, y eta, eta eta), 1, sl, 3 unused.
 constexpr int kCandG3 = 24;
 __device__ __forceinline__ void smooth_record3(const double* __restrict__ F, int npad, int i, double* __restrict__ o)
 {

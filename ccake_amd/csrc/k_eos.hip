@@ -540,7 +540,7 @@ __global__ __launch_bounds__(256) void k3_post(double* __restrict__ F, int npad,
     o[13] = col(CCAKE_F_SHV0 + 5) * isl2; o[14] = col(CCAKE_F_SHV0 + 6) * isl2; o[15] = col(CCAKE_F_SHV0 + 7) * isl2;
     o[16] = col(CCAKE_F_SHV0 + 10) * isl2; o[17] = col(CCAKE_F_SHV0 + 11) * isl2;
     o[18] = col(CCAKE_F_SHV0 + 15) * isl2;
-    o[19] = sl; o[20] = 0.0; o[21] = 0.0; o[22] = 0.0; o[23] = 0.0;
+    o[19] = 1.0; o[20] = sl; o[21] = 0.0; o[22] = 0.0; o[23] = 0.0;
   }
 }
 

@@ -22,13 +22,16 @@
 //   RK update            Evolver::step_rk (src/evolver.cpp:363-484), three positions and
 //                        three velocity components
 //
-// The pair kernels follow the 2+1D design: owner computes, a tile of 64
-// cell-sorted particles per wave, candidate records read wave-uniformly
-// into SGPRs, a tile's flattened candidate list cut into slices (one
-// single-wave workgroup each) whose partial sums a per-particle pass adds in
-// slice order.  A tile segment is the set of lanes in one (y, eta) cell row;
-// the cell rows within reach of its bounding box are walked as x runs.
+// The pair kernels are owner-computes without atomics, as in 2+1D, but in three
+// dimensions a tile of 64 targets reaches 3.4 times the volume of one target's
+// cutoff sphere (100,007 particles, 734 neighbours each), so at most 29 % of
+// its lanes would have a pair.  A tile is 16 cell-sorted targets (43 %): lane l
+// has target l % 16 and, of every four candidates, candidate l / 16.  A
+// workgroup of W waves shares a tile's candidates and adds its sums in LDS.
+// A tile segment is the set of targets in one (y, eta) cell row; the cell
+// rows within reach of its bounding box are walked as x runs.
 #include "pair_common.h"
+#include <type_traits>
 
 namespace ccake {
 
@@ -166,49 +169,106 @@ __device__ __forceinline__ void row_range3(const Grid& g, const Seg3& s, double 
   nrow = nry * (rz1 - rz0 + 1);
 }
 
-// Slice `slice` of `nslices` of a segment's flattened candidate list, rows
-// resolved 64 at a time lane-parallel (as for_spans_slice in 2+1D).  The
-// body runs on every lane (wave-uniform control flow, so the compiler keeps
-// one copy of the accumulators): it masks the lanes outside the segment
-// (`in` false) itself.
-template <class Body>
-__device__ __forceinline__ void for_spans_slice3(const Grid& g, const int32_t* __restrict__ cell_off,
-                                                 const Seg3& s, double rcs, int slice, int nslices, bool in,
-                                                 Body&& body)
+constexpr int kTile3 = 16;                            // targets of a tile
+constexpr int kGroups3 = kWave / kTile3;              // candidates of a step
+constexpr int kAhead3 = 4;                            // steps worked between two looks at the list
+constexpr int kList3 = kWave + kGroups3 * kAhead3;    // entries of a wave's list
+
+// What one lane of a wave wrote to LDS is there for the others.
+__device__ __forceinline__ void wave_sync()
+{
+#ifdef CCAKE_HOST_EMU
+  (void)__ballot(1);
+#else
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#endif
+}
+
+// Wave `slice` of a tile's W waves walks its share of a segment's candidates
+// (every W-th of the flattened list).  The list is taken in batches of 64, a
+// candidate per lane, as RunCursor does in 2+1D: the lanes find their
+// candidates' sorted indices, read NP doubles of their records, and those
+// within the cutoff of the segment's bounding box are put into the wave's
+// list in LDS: read(j, c) reads candidate j's entry (c[0..2] its position),
+// put(e, c, j) writes it at e, move(from, to) moves one entry.  work(e,
+// steps) does `steps` steps of four candidates from entry e on: kAhead3 at a
+// time while the list holds as many, one at a time at the end, where
+// pad(e) fills up the last four.  The next batch is read while a list is
+// worked.
+template <int W, int NP, class Read, class Put, class Move, class Pad, class Work>
+__device__ __forceinline__ void walk_tile3(const Grid& g, const int32_t* __restrict__ cell_off, const Seg3& seg,
+                                           double rc2, double rcs, int slice, Read&& read, Put&& put, Move&& move,
+                                           Pad&& pad, Work&& work)
 {
   const int lane = threadIdx.x & (kWave - 1);
+  const double far2 = rc2 * (1.0 + 1e-9);             // margin for rounding
   int ry0, nry, rz0, nrow;
-  row_range3(g, s, rcs, ry0, nry, rz0, nrow);
-  int tot = 0;
+  row_range3(g, seg, rcs, ry0, nry, rz0, nrow);
+  int fill = 0, base = 0;
   for (int r0 = 0; r0 < nrow; r0 += kWave) {
-    int b2, e2;
-    row_run3(g, cell_off, s, rcs, ry0, nry, rz0, nrow, r0 + lane, b2, e2);
-    tot += last_lane(wave_incl_scan_i(e2 - b2));
-  }
-  const int lo = (int)(((long long)tot * slice) / nslices);
-  const int hi = (int)(((long long)tot * (slice + 1)) / nslices);
-  int base = 0;
-  for (int r0 = 0; r0 < nrow && base < hi; r0 += kWave) {
-    int b, e;
-    row_run3(g, cell_off, s, rcs, ry0, nry, rz0, nrow, r0 + lane, b, e);
-    const int len = e - b;
-    const int incl = wave_incl_scan_i(len), pre = incl - len;
-    const int ctot = last_lane(incl);
-    const int nr = nrow - r0 < kWave ? nrow - r0 : kWave;
-    for (int r = 0; r < nr; ++r) {
-      const int rbase = base + __builtin_amdgcn_readlane(pre, r);
-      if (rbase >= hi) break;
-      const int rb = __builtin_amdgcn_readlane(b, r);
-      const int rlen = __builtin_amdgcn_readlane(len, r);
-      const int t0 = lo > rbase ? lo - rbase : 0;
-      const int t1 = hi - rbase < rlen ? hi - rbase : rlen;
-      if (t0 < t1) body(rb + t0, rb + t1);
+    int run, e;
+    row_run3(g, cell_off, seg, rcs, ry0, nry, rz0, nrow, r0 + lane, run, e);
+    const int len = e - run, incl = wave_incl_scan_i(len), first = base + incl - len;
+    const int end = base + last_lane(incl);
+    int t = base + slice, jn = 0;
+    bool vn = false;
+    double next[NP];
+    auto request = [&]() -> bool {
+      if (t >= end) return false;
+      const int q = t + W * lane;
+      vn = q < end;
+      jn = 0;
+      for (uint64_t m = __ballot(len > 0 && first < t + kWave * W && first + len > t); m; m &= m - 1) {
+        const int r = __builtin_ctzll(m);
+        const int f = __builtin_amdgcn_readlane(first, r), l = __builtin_amdgcn_readlane(len, r);
+        const int s = __builtin_amdgcn_readlane(run, r);
+        if (q >= f && q < f + l) jn = s + q - f;
+      }
+      read(jn, next);
+      t += kWave * W;
+      return true;
+    };
+    bool more = request();
+    while (more) {
+      double c[NP];
+      #pragma unroll
+      for (int q = 0; q < NP; ++q) c[q] = next[q];
+      const int j = jn;
+      double d2 = 0.0;
+      #pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double x = fmax(fmax(seg.mn[d] - c[d], c[d] - seg.mx[d]), 0.0);
+        d2 += x * x;
+      }
+      const bool keep = vn && d2 <= far2;
+      const uint64_t mask = __ballot(keep);
+      more = request();
+      if (keep) put(fill + __popcll(mask & ((1ull << lane) - 1)), c, j);
+      fill += __popcll(mask);
+      wave_sync();
+      int done = 0;
+      for (; fill - done >= kGroups3 * kAhead3; done += kGroups3 * kAhead3) work(done, std::integral_constant<int, kAhead3>());
+      if (done) {
+        wave_sync();
+        fill -= done;
+        if (lane < fill) move(done + lane, lane);
+        wave_sync();
+      }
     }
-    base += ctot;
+    base = end;
+  }
+  if (fill) {
+    const int whole = (fill + kGroups3 - 1) / kGroups3 * kGroups3;
+    if (lane >= fill && lane < whole) pad(lane);
+    wave_sync();
+    for (int e = 0; e < whole; e += kGroups3) work(e, std::integral_constant<int, 1>());
+    wave_sync();
   }
 }
 
-// Every candidate of a segment, one at a time (the count and export walks).
+// Every candidate of a segment, one at a time (the export walk).
 template <class Body>
 __device__ __forceinline__ void for_spans3(const Grid& g, const int32_t* __restrict__ cell_off, const Seg3& s,
                                            double rcs, Body&& body)
@@ -223,66 +283,6 @@ __device__ __forceinline__ void for_spans3(const Grid& g, const int32_t* __restr
   }
 }
 
-// Candidates j0 .. j1-1 one at a time, the next record requested while the
-// current one is evaluated (scalar loads; the wait falls after the current
-// arithmetic).  body(c, dx, dy, dz, j, valid).
-template <int NR, int STRIDE, class Body>
-__device__ __forceinline__ void walk_records3(const double* __restrict__ cand, const double* r, int j0, int j1,
-                                              Body&& body)
-{
-  if (j0 >= j1) return;
-  double cur[NR];
-  #pragma unroll
-  for (int q = 0; q < NR; ++q) cur[q] = cand[(size_t)j0 * STRIDE + q];
-  for (int j = j0; j < j1; ++j) {
-    const double dx = r[0] - cur[0], dy = r[1] - cur[1], dz = r[2] - cur[2];
-    __builtin_amdgcn_sched_barrier(0);
-    double nxt[NR];
-    const int jn = j + 1 < j1 ? j + 1 : j1 - 1;
-    #pragma unroll
-    for (int q = 0; q < NR; ++q) nxt[q] = cand[(size_t)jn * STRIDE + q];
-    __builtin_amdgcn_sched_barrier(0);
-    body(cur, dx, dy, dz, j, true);
-    #pragma unroll
-    for (int q = 0; q < NR; ++q) cur[q] = nxt[q];
-  }
-}
-
-// Candidates j0 .. j1-1 one at a time for records too large to double
-// buffer in SGPRs: the head of a record (position and mass, 4 doubles) is
-// requested one candidate ahead, the rest of it (entries 4 .. NR-1) when
-// its candidate comes up, together with the next head.  pair(c, dx, dy,
-// dz, w) computes the kernel factors w[3] from the head and returns false
-// when no lane has the pair in range (the rest is then not needed); sums(c,
-// w) adds the terms that need the rest.  The wait for the rest falls after
-// the kernel arithmetic, and 2*4 + NR - 4 doubles are in flight at most
-// (46 SGPRs for the 19-double shear record, against 76 for two records).
-template <int NR, int STRIDE, class Pair, class Sums>
-__device__ __forceinline__ void walk_records3_split(const double* __restrict__ cand, const double* r, int j0,
-                                                    int j1, Pair&& pair, Sums&& sums)
-{
-  if (j0 >= j1) return;
-  constexpr int NH = 4;
-  double head[NH];
-  #pragma unroll
-  for (int q = 0; q < NH; ++q) head[q] = cand[(size_t)j0 * STRIDE + q];
-  for (int j = j0; j < j1; ++j) {
-    double c[NR];
-    #pragma unroll
-    for (int q = 0; q < NH; ++q) c[q] = head[q];
-    const double dx = r[0] - c[0], dy = r[1] - c[1], dz = r[2] - c[2];
-    __builtin_amdgcn_sched_barrier(0);
-    const int jn = j + 1 < j1 ? j + 1 : j1 - 1;
-    #pragma unroll
-    for (int q = NH; q < NR; ++q) c[q] = cand[(size_t)j * STRIDE + q];
-    #pragma unroll
-    for (int q = 0; q < NH; ++q) head[q] = cand[(size_t)jn * STRIDE + q];
-    __builtin_amdgcn_sched_barrier(0);
-    double w[3];
-    if (pair(c, dx, dy, dz, w)) sums(c, w);
-  }
-}
-
 // Kernel constants of a 3+1D event.  Isotropic: W = norm2 w(q),
 // grad W = C rel g(q) with q = r / hT (SPHkernel<3>: norm2 = 1/(4 pi hT^3),
 // C = kgrad / hT^5 = -3/(4 pi hT^5)).  Factorized: W = norm2 w(q_perp) w(q_eta)
@@ -290,14 +290,12 @@ __device__ __forceinline__ void walk_records3_split(const double* __restrict__ c
 // 1/(6 hEta) the gradient is C (rel_x g_perp w_eta, rel_y g_perp w_eta,
 // kfac w_perp rel_eta g_eta), kfac = (5/(14 pi hT^2)) (-1/(2 hEta^3)) / C.
 struct Kern3 {
-  double norm2, C, kfac, hinv2, heinv2;
+  double norm2, C, kfac;
 };
 static Kern3 kern3(const ccake_params& p)
 {
   Kern3 k;
   const double h = p.hT, he = p.hEta;
-  k.hinv2 = 1.0 / (h * h);
-  k.heinv2 = he > 0.0 ? 1.0 / (he * he) : 0.0;
   if (p.factorized_kernel) {
     const double n2 = 5.0 / (14.0 * kPi) / (h * h), n1 = (1.0 / 6.0) / he;
     const double C2 = -15.0 / (14.0 * kPi) / pow(h, 4), C1 = -0.5 / pow(he, 3);
@@ -312,88 +310,147 @@ static Kern3 kern3(const ccake_params& p)
   return k;
 }
 
-// The weight w of one pair (W = norm2 w) for the isotropic or factorized
-// kernel; `nb` masks pairs outside the list (the factorized kernel can be
-// non-zero there when hEta > hT).
-template <bool FACT>
-__device__ __forceinline__ double pair_w3(double dx, double dy, double dz, double r2, bool nb, double hinv2,
-                                          double heinv2)
+// The tile and the target of this lane.
+struct Target3 {
+  int tile, slice, i, group, k;      // k: sorted position
+  bool act;
+};
+__device__ __forceinline__ Target3 target3(int n)
 {
-  if (FACT) {
-    double qp, iqp, qe, iqe;
-    q_and_inverse(dist2_perp(dx, dy), hinv2, qp, iqp);
-    q_and_inverse(dz * dz, heinv2, qe, iqe);
-    return nb ? spline_w(qp) * spline_w(qe) : 0.0;
-  } else {
-    double q, iq;
-    q_and_inverse(r2, hinv2, q, iq);
-    return nb ? spline_w(q) : 0.0;
-  }
+  Target3 t;
+  const int lane = threadIdx.x & (kWave - 1);
+  t.tile = xcd_tile(blockIdx.x, gridDim.x);
+  t.slice = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // wave-uniform
+  t.i = lane % kTile3;
+  t.group = lane / kTile3;
+  const int k = t.tile * kTile3 + t.i;
+  t.act = k < n;
+  t.k = t.act ? k : 0;
+  return t;
 }
 
 // ---------------------------------------------------------------------------
 // Smoothing, pair part: MODE 0 sigma_lab, s, B, S, Q and the neighbour count
-// (6 partial sums); MODE 1 sigma_lab and the count (initial sigma).  Same
-// partial-sum layout as the 2+1D kernel, so k_smooth_sum adds them.
-template <int MODE, bool FACT>
-__global__ __launch_bounds__(kWave) void k3_smooth_slice(const double* __restrict__ cand,
-                                                         const int32_t* __restrict__ skey,
-                                                         const int32_t* __restrict__ cell_off,
-                                                         const Grid* __restrict__ gridp, int n, double rc2,
-                                                         double rcs, double hinv2, double heinv2, int nslices,
-                                                         double* __restrict__ part, int npad)
+// (6 sums); MODE 1 sigma_lab and the count (initial sigma); MODE 2 the count
+// alone, written as btrack, and the pair total.  The sums go to `part` as
+// those of a single slice, so k_smooth_sum reads them.
+// Bound: the FP64 vector unit, 29 instructions per step of four candidates, and
+// the list's reads from LDS (32 of its cycles a step, four SIMDs a CU).  A
+// smoothing pass of 100,007 particles (73 M pairs): 363 us with 64 targets a
+// tile and records in scalar registers, 212 us now.  MODE 2 the same way: the
+// count walked one candidate at a time took 1.7 ms.
+template <int MODE, bool FACT, int W>
+__global__ __launch_bounds__(kWave * W) void k3_smooth_tile(const double* __restrict__ cand,
+                                                            const int32_t* __restrict__ skey,
+                                                            const int32_t* __restrict__ cell_off,
+                                                            const Grid* __restrict__ gridp, int n, double rc2,
+                                                            double rcs, double hinv, double heinv,
+                                                            double* __restrict__ part, int npad,
+                                                            const int32_t* __restrict__ perm,
+                                                            int32_t* __restrict__ btrack,
+                                                            unsigned long long* __restrict__ pair_total)
 {
-  constexpr int NACC = MODE == 0 ? 6 : 2;
+  constexpr int NACC = MODE == 0 ? 6 : (MODE == 1 ? 2 : 1);   // the count last
+  constexpr int NP = MODE == 0 ? 8 : 4;
+  __shared__ alignas(16) double list[W][kList3 * NP];
+  static_assert(kList3 * NP >= NACC * kWave, "the lists are reused for the sums");
   const Grid& g = *gridp;
-  const int lane = threadIdx.x;
-  const int unit = xcd_tile(blockIdx.x, gridDim.x);
-  const int tile = unit / nslices;
-  const int slice = unit - tile * nslices;
-  const int k = tile * kTile + lane;
-  const bool act = k < n;
-  const int kk = act ? k : 0;
-  const double* me = cand + (size_t)kk * kCandS;
+  const Target3 t = target3(n);
+  const double* me = cand + (size_t)t.k * kCandS;
   const double r[3] = { me[0], me[1], me[2] };
-  const int myrow = act ? skey[kk] / g.stride : INT_MAX;
+  const int myrow = t.act ? skey[t.k] / g.stride : INT_MAX;
+  const double m4h = -0.25 * hinv, mk2h = -0.5 * hinv * kSplineK;
+  double* mine = list[t.slice];
 
-  double sl = 0.0, ss = 0.0, sB = 0.0, sS = 0.0, sQ = 0.0;
+  double acc[5] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
   int cnt = 0;
-  for_segments3(act, myrow, r, [&](const Seg3& seg, bool in) {
-    for_spans_slice3(g, cell_off, seg, rcs, slice, nslices, in, [&](int j0, int j1) {
-      constexpr int NR = MODE == 0 ? 8 : 4;
-      walk_records3<NR, kCandS>(cand, r, j0, j1, [&](const double* c, double dx, double dy, double dz, int j,
-                                                     bool valid) {
-        const double r2 = dist2_3(dx, dy, dz);
-        const bool nb = in && valid && r2 <= rc2;
-        cnt += nb ? 1 : 0;
-        if (kSkipEmpty && wave_none(nb)) return;
-        const double w = pair_w3<FACT>(dx, dy, dz, r2, nb, hinv2, heinv2);
-        sl += c[3] * w;
-        if (MODE == 0) {
-          ss += c[MODE == 0 ? 4 : 0] * w; sB += c[MODE == 0 ? 5 : 0] * w;
-          sS += c[MODE == 0 ? 6 : 0] * w; sQ += c[MODE == 0 ? 7 : 0] * w;
+  for_segments3(t.act, myrow, r, [&](const Seg3& seg, bool in) {
+    const double xs = in ? r[0] : kFarAway;
+    walk_tile3<W, NP>(g, cell_off, seg, rc2, rcs, t.slice,
+      [&](int j, double (&c)[NP]) {
+        #pragma unroll
+        for (int q = 0; q < NP; ++q) c[q] = cand[(size_t)j * kCandS + q];
+      },
+      [&](int e, const double (&c)[NP], int) {
+        #pragma unroll
+        for (int q = 0; q < NP; ++q) mine[e * NP + q] = c[q];
+      },
+      [&](int from, int to) {
+        #pragma unroll
+        for (int q = 0; q < NP; ++q) mine[to * NP + q] = mine[from * NP + q];
+      },
+      [&](int e) {
+        mine[e * NP] = -kFarAway;
+        #pragma unroll
+        for (int q = 1; q < NP; ++q) mine[e * NP + q] = 0.0;
+      },
+      [&](int e0, auto steps) {
+        #pragma unroll
+        for (int u = 0; u < decltype(steps)::value; ++u) {
+          const double* c = mine + (e0 + kGroups3 * u + t.group) * NP;
+          const double dx = xs - c[0], dy = r[1] - c[1], dz = r[2] - c[2];
+          const double r2 = dist2_3(dx, dy, dz);
+          const bool nb = r2 <= rc2;
+          cnt += nb ? 1 : 0;
+          if (MODE == 2) continue;
+          double w;
+          if (FACT) {
+            double qp, iqp, qe, iqe;
+            q_and_inverse(dist2_perp(dx, dy), hinv * hinv, qp, iqp);
+            q_and_inverse(dz * dz, heinv * heinv, qe, iqe);
+            w = nb ? spline_w(qp) * spline_w(qe) : 0.0;
+          } else {
+            w = spline_w8(r2, m4h, mk2h);
+          }
+          acc[0] += c[3] * w;
+          if (MODE == 0) {
+            #pragma unroll
+            for (int q = 1; q < 5; ++q) acc[q] += c[MODE == 0 ? 3 + q : 0] * w;
+          }
         }
       });
-    });
   });
-  double* p = part + (size_t)slice * NACC * npad + k;
-  p[0] = sl;
-  p[(size_t)npad] = (double)cnt;
-  if (MODE == 0) {
-    p[(size_t)2 * npad] = ss; p[(size_t)3 * npad] = sB;
-    p[(size_t)4 * npad] = sS; p[(size_t)5 * npad] = sQ;
+  // the four groups of the W waves, in order
+  #pragma unroll
+  for (int q = 0; q < NACC - 1; ++q) mine[q * kWave + (threadIdx.x & (kWave - 1))] = FACT ? acc[q] : kSplineW * acc[q];
+  mine[(NACC - 1) * kWave + (threadIdx.x & (kWave - 1))] = (double)cnt;
+  __syncthreads();
+  unsigned long long tot = 0;
+  for (int o = threadIdx.x; o < NACC * kTile3; o += kWave * W) {
+    const int q = o / kTile3, i = o % kTile3;
+    double s = 0.0;
+    #pragma unroll
+    for (int w = 0; w < W; ++w)
+      #pragma unroll
+      for (int h = 0; h < kGroups3; ++h) s += list[w][q * kWave + h * kTile3 + i];
+    const int k = t.tile * kTile3 + i;
+    if (MODE == 2) {
+      if (k < n) {
+        // without the particle itself (counted unless its position is not finite)
+        const double* c = cand + (size_t)k * kCandS;
+        const int nb = (int)s - (dist2_3(c[0] - c[0], c[1] - c[1], c[2] - c[2]) <= rc2 ? 1 : 0);
+        const int id = perm[k];
+        tot = nb;
+        if (btrack[id] != -1) btrack[id] = nb;
+      }
+    } else {
+      // columns sigma_lab, count, s, B, S, Q
+      const int col = q == 0 ? 0 : (q == NACC - 1 ? 1 : q + 1);
+      part[(size_t)col * npad + k] = s;
+    }
+  }
+  if (MODE == 2 && pair_total && threadIdx.x < kWave) {
+    for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o);
+    if (threadIdx.x == 0) atomicAdd(pair_total, tot);
   }
 }
 
-// Neighbour walk without sums: MODE 2 counts (btrack) and the pair total;
-// MODE 3 writes the pair rows (parity export) at the row offsets.
-template <int MODE>
-__global__ __launch_bounds__(64) void k3_walk(const double* __restrict__ cand, const int32_t* __restrict__ skey,
-                                              const int32_t* __restrict__ perm, const int32_t* __restrict__ cell_off,
-                                              const Grid* __restrict__ gridp, int n, double rc2, double rcs,
-                                              int32_t* __restrict__ btrack, unsigned long long* __restrict__ pair_total,
-                                              const int64_t* __restrict__ row_off, int32_t* __restrict__ out_i,
-                                              int32_t* __restrict__ out_j)
+// The pair rows (parity export) at the row offsets.
+__global__ __launch_bounds__(64) void k3_export(const double* __restrict__ cand, const int32_t* __restrict__ skey,
+                                                const int32_t* __restrict__ perm, const int32_t* __restrict__ cell_off,
+                                                const Grid* __restrict__ gridp, int n, double rc2, double rcs,
+                                                const int64_t* __restrict__ row_off, int32_t* __restrict__ out_i,
+                                                int32_t* __restrict__ out_j)
 {
   const Grid& g = *gridp;
   const int lane = threadIdx.x;
@@ -404,160 +461,172 @@ __global__ __launch_bounds__(64) void k3_walk(const double* __restrict__ cand, c
   const double r[3] = { me[0], me[1], me[2] };
   const int myrow = act ? skey[kk] / g.stride : INT_MAX;
   const int id = act ? perm[kk] : 0;
-  int cnt = 0;
-  int64_t wpos = 0;
-  if (MODE == 3 && act) wpos = row_off[id];
+  int64_t wpos = act ? row_off[id] : 0;
   for_segments3(act, myrow, r, [&](const Seg3& seg, bool in) {
     for_spans3(g, cell_off, seg, rcs, [&](int j) {
       const double* c = cand + (size_t)j * kCandS;
       const double r2 = dist2_3(r[0] - c[0], r[1] - c[1], r[2] - c[2]);
-      const bool nb = in && (r2 <= rc2) && (j != k);
-      if (MODE == 2) cnt += nb;
-      if (MODE == 3 && nb) { out_i[wpos] = id; out_j[wpos] = perm[j]; ++wpos; }
+      if (in && (r2 <= rc2) && (j != k)) { out_i[wpos] = id; out_j[wpos] = perm[j]; ++wpos; }
     });
   });
-  if (MODE == 3) return;
-  unsigned long long tot = act ? (unsigned long long)cnt : 0ull;
-  for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o);
-  if (lane == 0 && pair_total) atomicAdd(pair_total, tot);
-  if (!act) return;
-  const int b = btrack[id];
-  btrack[id] = (b == -1) ? -1 : cnt;
 }
 
 // ---------------------------------------------------------------------------
-// Gradients, pair part.  With w = m_b grad W_ab / C the kernel accumulates
-// neighbour-side sums (as in 2+1D): sum w (3), (p_b/sl_b^2) w (3), e_b w (3),
-// (Pi_b/sl_b^2) w (3), v_b^j w_i (9) and, with shear, sum w.v_a (1),
-// (w.v_a) pi^{0j}_b/sl_b^2 (3), sum_i w_i pi^{ji}_b/sl_b^2 (3).
-template <bool SHEAR>
-constexpr int grad3_nacc() { return SHEAR ? 28 : 21; }
-
-// Register budget of the gradient walk: 4 waves per SIMD (128 VGPRs, a few
-// values spilled to scratch) measured 1.115 ms per launch on the 126k event
-// against 1.131 at 3 and 1.402 at the compiler's choice (183 VGPRs, 2 waves).
-#ifndef CCAKE_GRAD3_WAVES_PER_SIMD
-#define CCAKE_GRAD3_WAVES_PER_SIMD 4
-#endif
-template <bool SHEAR, bool FACT>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(CCAKE_GRAD3_WAVES_PER_SIMD)))
-void k3_grad_slice(const double* __restrict__ cand,
-                                                       const int32_t* __restrict__ skey,
-                                                       const int32_t* __restrict__ cell_off,
-                                                       const Grid* __restrict__ gridp, int n, double rc2, double rcs,
-                                                       double hinv2, double heinv2, double kfac, int nslices,
-                                                       double* __restrict__ part, int npad)
+// Gradients.  Of a candidate's record the kernel sums, per target and with
+// w_d = m_b d_d W_ab / C, the 3 x 16 products w_d f_j of the fields f_j =
+// (p/sl^2, e, Pi/sl^2, v (3), pi^{0i}/sl^2 (3), pi^{ij}/sl^2 (6), 1): a matrix
+// product of 16 targets by 16 fields over the candidates, which is what
+// v_mfma_f64_16x16x4 does four candidates at a time.  39 of the 48 are needed
+// (v_a is constant over b, so (w . v_a) pi^{0i} is a sum of them).
+// FP64 matrix instructions run at the vector unit's rate (65 cycles, against 39
+// vector instructions of 4), but each lane then needs one field of one
+// candidate, one coalesced load a step, where lanes of four candidates
+// would each read a whole record of 19 values; and the sums take 24 registers.
+// Bound: the FP64 unit, 24 vector instructions and three matrix instructions
+// (300 cycles) a step.  Gradients of 100,007 particles: 890 us with 64 targets a
+// tile, vector sums and a sum pass over the slices, 390 us now.
+typedef double Sums3 __attribute__((vector_size(4 * sizeof(double))));   // targets group + 4 r, field lane % 16
+__device__ __forceinline__ void outer3(const double (&w)[3], double f, Sums3 (&acc)[3])
 {
-  constexpr int NACC = grad3_nacc<SHEAR>();
-  const Grid& g = *gridp;
-  const int lane = threadIdx.x;
-  const int unit = xcd_tile(blockIdx.x, gridDim.x);
-  const int tile = unit / nslices;
-  const int slice = unit - tile * nslices;
-  const int k = tile * kTile + lane;
-  const bool act = k < n;
-  const int kk = act ? k : 0;
-  const double* me = cand + (size_t)kk * kCandG3;
-  const double r[3] = { me[0], me[1], me[2] };
-  const double va[3] = { me[7], me[8], me[9] };
-  const int myrow = act ? skey[kk] / g.stride : INT_MAX;
-
-  double acc[NACC];
+#ifdef CCAKE_HOST_EMU
+  __shared__ double s[8][4][kWave];
+  const int lane = threadIdx.x % kWave;
+  auto& mine = s[threadIdx.x / kWave];
+  for (int d = 0; d < 3; ++d) mine[d][lane] = w[d];
+  mine[3][lane] = f;
+  wave_sync();
+  for (int d = 0; d < 3; ++d)
+    for (int r = 0; r < 4; ++r)
+      for (int k = 0; k < kGroups3; ++k)
+        acc[d][r] += mine[d][lane / kTile3 + 4 * r + kTile3 * k] * mine[3][lane % kTile3 + kTile3 * k];
+  wave_sync();
+#else
   #pragma unroll
-  for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
-  for_segments3(act, myrow, r, [&](const Seg3& seg, bool in) {
-    for_spans_slice3(g, cell_off, seg, rcs, slice, nslices, in, [&](int j0, int j1) {
-      constexpr int NR = SHEAR ? 19 : 10;
-      auto pair = [&](const double* c, double dx, double dy, double dz, double* w) -> bool {
-        const double r2 = dist2_3(dx, dy, dz);
-        const bool nb = in && r2 <= rc2;
-        if (kSkipEmpty && wave_none(nb)) return false;
-        if (FACT) {
-          double qp, iqp, qe, iqe;
-          q_and_inverse(dist2_perp(dx, dy), hinv2, qp, iqp);
-          q_and_inverse(dz * dz, heinv2, qe, iqe);
-          const double m = nb ? c[3] : 0.0;
-          const double gp = m * spline_g(qp, iqp) * spline_w(qe);
-          w[0] = gp * dx; w[1] = gp * dy;
-          w[2] = m * kfac * spline_w(qp) * spline_g(qe, iqe) * dz;
-        } else {
-          double q, iq;
-          q_and_inverse(r2, hinv2, q, iq);
-          const double gm = nb ? c[3] * spline_g(q, iq) : 0.0;
-          w[0] = gm * dx; w[1] = gm * dy; w[2] = gm * dz;
-        }
-        return true;
-      };
-      auto sums = [&](const double* c, const double* w) {
-        #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          acc[d] += w[d];
-          acc[3 + d] += c[4] * w[d];
-          acc[6 + d] += c[5] * w[d];
-          acc[9 + d] += c[6] * w[d];
-          #pragma unroll
-          for (int e = 0; e < 3; ++e) acc[12 + 3 * d + e] += c[7 + e] * w[d];
-        }
-        if (SHEAR) {
-          const double cv = w[0] * va[0] + w[1] * va[1] + w[2] * va[2];
-          acc[SHEAR ? 21 : 0] += cv;
-          #pragma unroll
-          for (int e = 0; e < 3; ++e) acc[SHEAR ? 22 + e : 0] += cv * c[SHEAR ? 10 + e : 0];
-          // pi^{ji}, i summed with w_i: rows of (xx, xy, x eta; xy, yy, y eta; x eta, y eta, eta eta)
-          acc[SHEAR ? 25 : 0] += w[0] * c[SHEAR ? 13 : 0] + w[1] * c[SHEAR ? 14 : 0] + w[2] * c[SHEAR ? 15 : 0];
-          acc[SHEAR ? 26 : 0] += w[0] * c[SHEAR ? 14 : 0] + w[1] * c[SHEAR ? 16 : 0] + w[2] * c[SHEAR ? 17 : 0];
-          acc[SHEAR ? 27 : 0] += w[0] * c[SHEAR ? 15 : 0] + w[1] * c[SHEAR ? 17 : 0] + w[2] * c[SHEAR ? 18 : 0];
-        }
-      };
-      walk_records3_split<NR, kCandG3>(cand, r, j0, j1, pair, sums);
-    });
-  });
-  double* p = part + (size_t)slice * NACC * npad + k;
-  #pragma unroll
-  for (int q = 0; q < NACC; ++q) p[(size_t)q * npad] = acc[q];
+  for (int d = 0; d < 3; ++d) acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[d], f, acc[d], 0, 0, 0);
+#endif
 }
 
-// Sum pass: the slices in slice order, scaled by C, then the owner terms
-// (from the particle's own record), written by particle id.
-template <bool SHEAR>
-__global__ __launch_bounds__(256) void k3_grad_sum(const double* __restrict__ cand, const int32_t* __restrict__ perm,
-                                                   int n, double C, const double* __restrict__ part, int nslices,
-                                                   int npad, double* __restrict__ F)
+template <bool SHEAR, bool FACT, int W>
+__global__ __launch_bounds__(kWave * W) void k3_grad_tile(const double* __restrict__ cand,
+                                                          const int32_t* __restrict__ skey,
+                                                          const int32_t* __restrict__ cell_off,
+                                                          const Grid* __restrict__ gridp, int n, double rc2,
+                                                          double rcs, double hinv, double heinv, double kfac, double C,
+                                                          const int32_t* __restrict__ perm, int npad,
+                                                          double* __restrict__ F)
 {
-  constexpr int NACC = grad3_nacc<SHEAR>();
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  double acc[NACC];
+  constexpr int NSUM = 3 * 16 * kTile3;               // a wave's sums: [direction][field][target]
+  constexpr int NP = 4;                               // x, y, eta, m
+  static_assert(NSUM >= kList3 * (NP + 1), "the lists are reused for the sums");
+  __shared__ alignas(16) double buf[W][NSUM];
+  const Grid& g = *gridp;
+  const Target3 t = target3(n);
+  const int lane = threadIdx.x & (kWave - 1);
+  const double* me = cand + (size_t)t.k * kCandG3;
+  const double r[3] = { me[0], me[1], me[2] };
+  const int myrow = t.act ? skey[t.k] / g.stride : INT_MAX;
+  const double m4h = -0.25 * hinv, m2h = -0.5 * hinv;
+  double* pos = buf[t.slice];
+  long long* off = reinterpret_cast<long long*>(buf[t.slice] + kList3 * NP);   // a record's first field
+  const double* fields = cand + 4 + t.i;
+
+  Sums3 acc[3] = { { 0.0, 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0, 0.0 } };
+  for_segments3(t.act, myrow, r, [&](const Seg3& seg, bool in) {
+    const double xs = in ? r[0] : kFarAway;
+    walk_tile3<W, NP>(g, cell_off, seg, rc2, rcs, t.slice,
+      [&](int j, double (&c)[NP]) {
+        #pragma unroll
+        for (int q = 0; q < NP; ++q) c[q] = cand[(size_t)j * kCandG3 + q];
+      },
+      [&](int e, const double (&c)[NP], int j) {
+        #pragma unroll
+        for (int q = 0; q < NP; ++q) pos[e * NP + q] = c[q];
+        off[e] = (long long)j * kCandG3;
+      },
+      [&](int from, int to) {
+        #pragma unroll
+        for (int q = 0; q < NP; ++q) pos[to * NP + q] = pos[from * NP + q];
+        off[to] = off[from];
+      },
+      [&](int e) {
+        pos[e * NP] = -kFarAway;
+        #pragma unroll
+        for (int q = 1; q < NP; ++q) pos[e * NP + q] = 0.0;
+        off[e] = off[0];
+      },
+      [&](int e0, auto steps) {
+        constexpr int U = decltype(steps)::value;
+        double f[U];
+        #pragma unroll
+        for (int u = 0; u < U; ++u) f[u] = fields[off[e0 + kGroups3 * u + t.group]];
+        #pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const double* c = pos + (e0 + kGroups3 * u + t.group) * NP;
+          const double dx = xs - c[0], dy = r[1] - c[1], dz = r[2] - c[2];
+          double w[3];
+          if (FACT) {
+            double qp, iqp, qe, iqe;
+            q_and_inverse(dist2_perp(dx, dy), hinv * hinv, qp, iqp);
+            q_and_inverse(dz * dz, heinv * heinv, qe, iqe);
+            const double m = dist2_3(dx, dy, dz) <= rc2 ? c[3] : 0.0;
+            const double gp = m * spline_g(qp, iqp) * spline_w(qe);
+            w[0] = gp * dx; w[1] = gp * dy;
+            w[2] = m * kfac * spline_w(qp) * spline_g(qe, iqe) * dz;
+          } else {
+            const double gm = c[3] * spline_g2(fma(dx, dx, fma(dy, dy, dz * dz)), m4h, m2h);
+            w[0] = gm * dx; w[1] = gm * dy; w[2] = gm * dz;
+          }
+          outer3(w, f[u], acc);
+        }
+      });
+  });
   #pragma unroll
-  for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
-  for (int sli = 0; sli < nslices; ++sli)
+  for (int d = 0; d < 3; ++d)
     #pragma unroll
-    for (int q = 0; q < NACC; ++q) acc[q] += part[((size_t)sli * NACC + q) * npad + k];
-  #pragma unroll
-  for (int q = 0; q < NACC; ++q) acc[q] *= C;
-  const double* me = cand + (size_t)k * kCandG3;
+    for (int q = 0; q < 4; ++q) buf[t.slice][(d * 16 + lane % 16) * kTile3 + lane / 16 + 4 * q] = acc[d][q];
+  __syncthreads();
+  if (W > 1) {
+    for (int o = threadIdx.x; o < NSUM; o += kWave * W) {
+      double s = buf[0][o];
+      #pragma unroll
+      for (int w = 1; w < W; ++w) s += buf[w][o];
+      buf[0][o] = s;
+    }
+    __syncthreads();
+  }
+  // the owner terms, a thread per target and direction, by particle id
+  const int i = threadIdx.x % kTile3, d = threadIdx.x / kTile3, k = t.tile * kTile3 + i;
+  if (d >= 3 || k >= n) return;
+  const double scale = FACT ? C : C * (2.0 / hinv);   // spline_g = 2 h spline_g2
+  auto sum = [&](int dir, int field) { return scale * buf[0][(dir * 16 + field) * kTile3 + i]; };
+  const double* own = cand + (size_t)k * kCandG3;
   const int id = perm[k];
   auto put = [&](int c, double v) { F[(size_t)c * npad + id] = v; };
-  const double sla = me[19], isla = 1.0 / sla;
+  const double sla = own[20], isla = 1.0 / sla;
+  const double s1 = sum(d, 15);                       // sum w_d
+  put(CCAKE_F_GRADP0 + d, sla * (sum(d, 0) + own[4] * s1));
+  put(CCAKE_F_GRADE0 + d, (sum(d, 1) - own[5] * s1) * isla);
+  put(CCAKE_F_GRADBULK0 + d, sla * (sum(d, 2) + own[6] * s1));
   #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    put(CCAKE_F_GRADP0 + d, sla * (acc[3 + d] + me[4] * acc[d]));
-    put(CCAKE_F_GRADE0 + d, (acc[6 + d] - me[5] * acc[d]) * isla);
-    put(CCAKE_F_GRADBULK0 + d, sla * (acc[9 + d] + me[6] * acc[d]));
-    #pragma unroll
-    for (int e = 0; e < 3; ++e) put(CCAKE_F_GRADV0 + 3 * d + e, (acc[12 + 3 * d + e] - me[7 + e] * acc[d]) * isla);
-  }
+  for (int e = 0; e < 3; ++e) put(CCAKE_F_GRADV0 + 3 * d + e, (sum(d, 3 + e) - own[7 + e] * s1) * isla);
+  double gs = 0.0, ds = 0.0;
   if (SHEAR) {
-    const double acv = acc[SHEAR ? 21 : 0];
+    double cv = 0.0, c0 = 0.0, ci = 0.0, oi = 0.0;
     #pragma unroll
-    for (int e = 0; e < 3; ++e) put(CCAKE_F_GRADSHEAR0 + e, sla * (acc[SHEAR ? 22 + e : 0] + me[10 + e] * acv));
-    // pi_a^{ji} a1_i with pi_a = (xx, xy, x eta, yy, y eta, eta eta) at me[13..18]
-    put(CCAKE_F_DIVSHEAR0 + 0, sla * (acc[SHEAR ? 25 : 0] + me[13] * acc[0] + me[14] * acc[1] + me[15] * acc[2]));
-    put(CCAKE_F_DIVSHEAR0 + 1, sla * (acc[SHEAR ? 26 : 0] + me[14] * acc[0] + me[16] * acc[1] + me[17] * acc[2]));
-    put(CCAKE_F_DIVSHEAR0 + 2, sla * (acc[SHEAR ? 27 : 0] + me[15] * acc[0] + me[17] * acc[1] + me[18] * acc[2]));
-  } else {
-    for (int e = 0; e < 3; ++e) { put(CCAKE_F_GRADSHEAR0 + e, 0.0); put(CCAKE_F_DIVSHEAR0 + e, 0.0); }
+    for (int a = 0; a < 3; ++a) {
+      const double s = sum(a, 15);
+      cv += s * own[7 + a];                           // sum w . v_a
+      c0 += sum(a, 6 + d) * own[7 + a];               // sum (w . v_a) pi^{0d}
+      // pi^{da}: (xx, xy, x eta, yy, y eta, eta eta)
+      const int q = d < a ? d : a, p = 9 + q * (5 - q) / 2 + (d < a ? a : d);
+      ci += sum(a, p);
+      oi += own[4 + p] * s;
+    }
+    gs = sla * (c0 + own[10 + d] * cv);
+    ds = sla * (ci + oi);
   }
+  put(CCAKE_F_GRADSHEAR0 + d, gs);
+  put(CCAKE_F_DIVSHEAR0 + d, ds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1060,33 +1129,34 @@ double smooth_norm2_event(const ccake_event* ev)
   return smooth_norm2(ev->p.hT);
 }
 
+// Waves per tile: the event's slices, as far as there are variants.
+static int tile3_waves(const ccake_event* ev) { return ev->nslices >= 4 ? 4 : (ev->nslices >= 2 ? 2 : 1); }
+
 int launch3_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
 {
   const int n = ev->n;
-  ev->smooth_sum_slices = ev->nslices;
+  ev->smooth_sum_slices = 1;
   const double rc = 2.0 * ev->p.hT;
-  const double rc2 = rc * rc;
-  const double rcs = search_radius(ev);
-  const int ntiles = (n + kTile - 1) / kTile;
-  hipStream_t st = ev->stream;
-  if (mode == 2) {
-    int32_t* bt = ev->I + (size_t)CCAKE_I_BTRACK * ev->npad;
-    unsigned long long* pc = count_pairs ? (unsigned long long*)ev->pair_count : nullptr;
-    hipLaunchKernelGGL(k3_walk<2>, dim3(ntiles), dim3(kTile), 0, st, ev->cand_s, ev->skey, ev->perm, ev->cell_off,
-                       ev->grid, n, rc2, rcs, bt, pc, nullptr, nullptr, nullptr);
-    return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
-  }
-  const Kern3 K = kern3(ev->p);
-  const dim3 grid(ntiles * ev->nslices), blk(kWave);
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, blk, 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n, rc2, rcs, K.hinv2,
-                       K.heinv2, ev->nslices, ev->part, ev->npad);
+  const double hinv = 1.0 / ev->p.hT, heinv = ev->p.hEta > 0.0 ? 1.0 / ev->p.hEta : 0.0;
+  unsigned long long* pc = mode == 2 && count_pairs ? (unsigned long long*)ev->pair_count : nullptr;
+  auto go = [&](auto kern, int W) {
+    hipLaunchKernelGGL(kern, dim3((n + kTile3 - 1) / kTile3), dim3(kWave * W), 0, ev->stream, ev->cand_s, ev->skey,
+                       ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), hinv, heinv, ev->part, ev->npad, ev->perm,
+                       ev->I + (size_t)CCAKE_I_BTRACK * ev->npad, pc);
   };
-  if (ev->p.factorized_kernel) {
-    if (mode == 0) go(k3_smooth_slice<0, true>); else go(k3_smooth_slice<1, true>);
-  } else {
-    if (mode == 0) go(k3_smooth_slice<0, false>); else go(k3_smooth_slice<1, false>);
-  }
+  auto waves = [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    if (mode == 2) go(k3_smooth_tile<2, false, W>, W);
+    else if (ev->p.factorized_kernel) {
+      if (mode == 0) go(k3_smooth_tile<0, true, W>, W); else go(k3_smooth_tile<1, true, W>, W);
+    } else {
+      if (mode == 0) go(k3_smooth_tile<0, false, W>, W); else go(k3_smooth_tile<1, false, W>, W);
+    }
+  };
+  const int W = tile3_waves(ev);
+  if (W == 4) waves(std::integral_constant<int, 4>());
+  else if (W == 2) waves(std::integral_constant<int, 2>());
+  else waves(std::integral_constant<int, 1>());
   return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
 }
 
@@ -1121,10 +1191,10 @@ int launch3_export_pairs(ccake_event* ev, int32_t* pi, int32_t* pj, size_t cap, 
   int32_t* d_j = static_cast<int32_t*>(b_j.p);
   CCAKE_HIP(hipMemcpyAsync(d_off, off.data(), (n + 1) * sizeof(int64_t), hipMemcpyHostToDevice, st));
   const double rc = 2.0 * ev->p.hT;
-  hipLaunchKernelGGL(k3_walk<3>, dim3((n + kTile - 1) / kTile), dim3(kTile), 0, st, ev->cand_s, ev->skey, ev->perm,
-                     ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), bt, nullptr, d_off, d_i, d_j);
+  hipLaunchKernelGGL(k3_export, dim3((n + kTile - 1) / kTile), dim3(kTile), 0, st, ev->cand_s, ev->skey, ev->perm,
+                     ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), d_off, d_i, d_j);
   const hipError_t le = hipGetLastError();
-  if (le != hipSuccess) { (void)hipStreamSynchronize(st); return hip_fail(le, "k3_walk"); }
+  if (le != hipSuccess) { (void)hipStreamSynchronize(st); return hip_fail(le, "k3_export"); }
   CCAKE_HIP(hipMemcpyAsync(pi, d_i, total * sizeof(int32_t), hipMemcpyDeviceToHost, st));
   CCAKE_HIP(hipMemcpyAsync(pj, d_j, total * sizeof(int32_t), hipMemcpyDeviceToHost, st));
   CCAKE_HIP(hipStreamSynchronize(st));
@@ -1136,28 +1206,25 @@ int launch3_grad(ccake_event* ev)
 {
   const int n = ev->n;
   const double rc = 2.0 * ev->p.hT;
-  const double rcs = search_radius(ev);
+  const double hinv = 1.0 / ev->p.hT, heinv = ev->p.hEta > 0.0 ? 1.0 / ev->p.hEta : 0.0;
   const Kern3 K = kern3(ev->p);
-  const int ntiles = (n + kTile - 1) / kTile;
-  hipStream_t st = ev->stream;
-  const dim3 grid(ntiles * ev->nslices), blk(kWave);
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, blk, 0, st, ev->cand_g, ev->skey, ev->cell_off, ev->grid, n, rc * rc, rcs,
-                       K.hinv2, K.heinv2, K.kfac, ev->nslices, ev->part, ev->npad);
-  };
-  const bool shear = ev->p.using_shear != 0;
-  if (shear) {
-    if (ev->p.factorized_kernel) go(k3_grad_slice<true, true>); else go(k3_grad_slice<true, false>);
-  } else {
-    if (ev->p.factorized_kernel) go(k3_grad_slice<false, true>); else go(k3_grad_slice<false, false>);
-  }
-  const dim3 g2((n + 255) / 256), b2(256);
-  if (shear)
-    hipLaunchKernelGGL(k3_grad_sum<true>, g2, b2, 0, st, ev->cand_g, ev->perm, n, K.C, ev->part, ev->nslices, ev->npad,
+  auto go = [&](auto kern, int W) {
+    hipLaunchKernelGGL(kern, dim3((n + kTile3 - 1) / kTile3), dim3(kWave * W), 0, ev->stream, ev->cand_g, ev->skey,
+                       ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), hinv, heinv, K.kfac, K.C, ev->perm, ev->npad,
                        ev->F);
-  else
-    hipLaunchKernelGGL(k3_grad_sum<false>, g2, b2, 0, st, ev->cand_g, ev->perm, n, K.C, ev->part, ev->nslices,
-                       ev->npad, ev->F);
+  };
+  auto waves = [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    if (ev->p.using_shear) {
+      if (ev->p.factorized_kernel) go(k3_grad_tile<true, true, W>, W); else go(k3_grad_tile<true, false, W>, W);
+    } else {
+      if (ev->p.factorized_kernel) go(k3_grad_tile<false, true, W>, W); else go(k3_grad_tile<false, false, W>, W);
+    }
+  };
+  const int W = tile3_waves(ev);
+  if (W == 4) waves(std::integral_constant<int, 4>());
+  else if (W == 2) waves(std::integral_constant<int, 2>());
+  else waves(std::integral_constant<int, 1>());
   return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
 }
 

@@ -348,6 +348,9 @@ inline int choose_slices(int ntiles, int simds)
 // particles, 41 tiles: smoothing and gradients 55 us a stage with 8, 58 with
 // 16), and 16 cost where they do not (30,300 particles: 128 against 142 us).
 constexpr int kTileWaves = 8;
+// 3+1D, tiles of 16 targets: smoothing and gradients 662 us a stage with 1 wave,
+// 608 with 2, 602 with 4 at 100,007 particles; 172, 146 and 134 at 25,018.
+constexpr int kTileWaves3 = 4;
 // The gradient walk's waves are longer: 4 once they fill the SIMDs (188,250
 // particles, 2,942 tiles: 965 us with 4, 974 with 8; 182,355 in six events:
 // 349 against 369; 40,401 particles, 632 tiles: 96 us with 4, 89 with 8).

@@ -9,6 +9,7 @@ import ccake_amd  # noqa: F401
 from ccake_amd import config
 from parity_metrics import DERIVS, STATE
 from test_gpu_parity import Pair, compare, ints_equal
+from test_milne3 import DERIVS3, STATE3, Pair3, compare3
 
 pytestmark = pytest.mark.gpu
 
@@ -41,4 +42,34 @@ def test_walk_edges(dev, orc, n, half, cells, particlization, shear):
     p.step(1)
     ints_equal(p.g, p.o, "BTRACK")
     compare(p.g, p.o, STATE + DERIVS, what=f"n={n} cells={cells} surface={particlization} shear={shear}")
+    p.close()
+
+
+# 3+1D: tiles of 16 targets; one particle, a tile and its neighbours, several
+# cell rows in a tile (1 and 8 cells per radius), 24 cells per radius (more than
+# 64 cell rows within reach), each number of waves per tile, both kernels, with
+# and without the shear sums
+@pytest.mark.parametrize("n,cells,waves,factorized,shear", [
+    (1, 2, 4, 0, 1), (15, 2, 2, 0, 1), (16, 2, 1, 1, 1), (17, 1, 4, 0, 0), (70, 8, 4, 1, 1), (343, 24, 4, 0, 1),
+    (1000, 2, 1, 0, 1), (1000, 2, 2, 1, 0), (1000, 2, 4, 0, 0), (1331, 3, 4, 1, 1)])
+def test_milne_walk_edges(dev, orc, n, cells, waves, factorized, shear):
+    m = int(np.ceil(round(n ** (1 / 3), 9)))
+    rng = np.random.default_rng(n)
+    g = (np.arange(m) - 0.5 * (m - 1)) * 0.17
+    x, y, eta = (a.ravel()[:n] + rng.uniform(-0.02, 0.02, n) for a in np.meshgrid(g, g, g))
+    e = (5.0 + 20.0 * np.exp(-(x * x + y * y + eta * eta) / 2.0)) / config.HBARC_GEVFM
+    f = 0.02 * np.cos(x + 0.3 * y)
+    d = dict(x=x, y=y, eta=eta, e=e, ux=0.1 * x, uy=-0.05 * y, ueta=0.03 * eta, rhoB=f * e, rhoS=0.5 * f * e, rhoQ=-f * e)
+    cfg = config.base_params(dim=3, hEta=0.2, factorized_kernel=factorized, t0=0.6, dt=0.01, particlization=0,
+                             eta_mode=config.ETA_CONSTANT, constant_eta_over_s=0.08 if shear else 0.0,
+                             cells_per_rc=cells, x_subcells=4)
+    p = Pair3(dev, orc, cfg, d)
+    p.g.nslices(waves)
+    p.g.initialize()
+    assert p.o.initialize() == 0
+    ints_equal(p.g, p.o, "BTRACK")
+    p.g.advance_timestep(cfg["dt"], 2)
+    assert p.o.advance_timestep(cfg["dt"], 2) == 0
+    ints_equal(p.g, p.o, "BTRACK")
+    compare3(p.g, p.o, STATE3 + DERIVS3, what=f"n={n} cells={cells} waves={waves} factorized={factorized} shear={shear}")
     p.close()
