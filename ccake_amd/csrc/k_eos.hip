@@ -369,7 +369,11 @@ static Transport make_transport(const ccake_params& p)
 #define CCAKE_EOS_THREADS 64
 #endif
 constexpr int kEosThreads = CCAKE_EOS_THREADS;
-constexpr int kHardWaves = 512;     // waves of k_eos_hard, striding over the hard list
+// Waves of k_eos_hard, striding over the hard list: two per SIMD, what its
+// registers allow.  A time step's list is empty or short (4.7 us with 512 or
+// 2,048 waves), the initial inversion's is long where the seed is far from
+// the root (40,401 particles of a Gubser event: 340 us with 512, 136 with 2,048).
+constexpr int kHardWaves = 2048;
 constexpr int kConformalChain = (1 << M_CONF) | (1 << M_DIAG);
 
 static int chain_kinds(const EosChain& ch)
