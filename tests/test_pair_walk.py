@@ -4,6 +4,7 @@ other parity tests: sums of at most a few thousand FP64 terms in another
 order)."""
 import numpy as np
 import pytest
+from scipy.spatial import cKDTree
 
 import ccake_amd  # noqa: F401
 from ccake_amd import config
@@ -73,3 +74,23 @@ def test_milne_walk_edges(dev, orc, n, cells, waves, factorized, shear):
     ints_equal(p.g, p.o, "BTRACK")
     compare3(p.g, p.o, STATE3 + DERIVS3, what=f"n={n} cells={cells} waves={waves} factorized={factorized} shear={shear}")
     p.close()
+
+
+# the cell sort: radix blocks of 1,024 (one, a partial one, 17 over the scan's 16
+# waves, the most its one workgroup takes and one more) and runs of empty cells
+@pytest.mark.parametrize("n", [1, 1023, 1025, 16385, 17409, 262144, 262145])
+def test_sort_and_counts(dev, n):
+    rng = np.random.default_rng(n)
+    half = max(1.0, 0.12 * np.sqrt(n))
+    r = rng.uniform(-half, half, (n, 2))
+    r[r[:, 0] > 0.0, 0] += 3.0 * half                 # two clouds with empty cells between
+    cfg = config.base_params(t0=0.6, dt=0.01, particlization=0, cells_per_rc=1, x_subcells=1)
+    eos = ccake_amd.Eos(dev, 0, 0.75)
+    ev = ccake_amd.Event(dev, eos, cfg, n)
+    ev.upload("CCAKE_F_X", r[:, 0])
+    ev.upload("CCAKE_F_Y", r[:, 1])
+    ev.build_neighbors()
+    want = cKDTree(r).query_ball_point(r, 2.0 * cfg["hT"], return_length=True) - 1
+    assert np.array_equal(ev.download_int("CCAKE_I_BTRACK"), want)
+    ev.close()
+    eos.close()
