@@ -296,7 +296,7 @@ def timed_steps(dev, eos, d, cfg, warmup, steps):
 
 def mixed_precision(dev, eos, d, cfg, warmup, steps, fp64_ms, fp64_event, fp64_rows):
     """The same workload with the mixed-precision pair sums (pair_precision
-    1: FP32 pair terms, compensated FP32 accumulation, FP64 elsewhere):
+    1: single-precision pair weights, FP64 sums and everything else):
     step time, the whole event to freeze-out, and the per-field error of its
     freeze-out hypersurface against the FP64 run's (rows matched by particle
     id; ccake_amd.precision gives the measures)."""

@@ -20,8 +20,7 @@ namespace ccake {
 
 // The walk of one (tile, slice) unit: slice `slice` of `nslices` of the
 // tile's candidates, one wave; fin(acc) receives the neighbour-side sums of
-// m_b grad W / C, summed as spline_g2 m_b rel and scaled by its 2 h at the end
-// (KEEP: with the arithmetic of q_and_inverse and spline_g, keep_order).
+// m_b grad W / C, summed as spline_g2 m_b rel and scaled by its 2 h at the end.
 // BULK false: the event's bulk pressure is zero on every particle (zeta = 0
 // and no initial bulk, checked at initialize), so the grad Pi sums are the
 // exact zeros the full walk would give and are not accumulated.
@@ -31,12 +30,13 @@ namespace ccake {
 // cycles, a vector instruction 4), so the sums stay on the vector side.
 // 188,250 particles (479M pairs): 1.30 ms per launch with 50 instructions
 // and no request ahead, 0.96 ms now.
-template <bool SHEAR, bool BULK, bool KEEP, class Fin>
+template <bool SHEAR, bool BULK, int FORM, class Fin>
 __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const int32_t* __restrict__ skey,
                                           const int32_t* __restrict__ cell_off, const Grid* __restrict__ gridp,
                                           int n, double rc2, double rcs, double hinv2, double m4h, double m2h, int tile, int slice,
                                           int nslices, Fin&& fin)
 {
+  constexpr bool KEEP = FORM == kKeep;
   const Grid& g0 = *gridp;
   const int lane = threadIdx.x & (kWave - 1);
   const int k = tile * kTile + lane;
@@ -67,7 +67,7 @@ __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const
           q_and_inverse(r2, hinv2, q, iq);
           gm = c[2] * spline_g(q, iq);
         } else {
-          gm = c[2] * spline_g2(r2, m4h, m2h);
+          gm = c[2] * spline_g2<FORM>(r2, m4h, m2h);
         }
         const double wx = gm * dx, wy = gm * dy;
         acc[0] += wx; acc[1] += wy;                    // sum m_b grad W
@@ -92,7 +92,7 @@ __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const
     });
   });
   if (!KEEP) {
-    const double h2 = -1.0 / m2h;
+    const double h2 = (FORM == kSingle ? -4.0 : -1.0) / m2h;
     #pragma unroll
     for (int q = 0; q < NW; ++q) acc[q] *= h2;
   }
@@ -112,7 +112,7 @@ __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const
 // Pair part: one single-wave workgroup per (tile, slice) unit walks its
 // slice of the tile's candidates and stores the slice's neighbour-side sums;
 // k_grad_sum adds the slices in slice order and applies the owner terms.
-template <bool SHEAR, bool BULK>
+template <bool SHEAR, bool BULK, int FORM = kExact>
 __global__ __launch_bounds__(kWave) void k_grad_slice(const double* __restrict__ cand,
                                                       const int32_t* __restrict__ skey,
                                                       const int32_t* __restrict__ cell_off,
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kWave) void k_grad_slice(const double* __restrict__
   const int unit = xcd_tile(blockIdx.x, gridDim.x);
   const int tile = unit / nslices;
   const int slice = unit - tile * nslices;
-  grad_walk<SHEAR, BULK, false>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, m2h, tile, slice, nslices,
+  grad_walk<SHEAR, BULK, FORM>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, m2h, tile, slice, nslices,
                          [&](const double* acc) {
     double* p = part + (size_t)slice * NACC * npad + tile * kTile + threadIdx.x;
     for (int q = 0; q < NACC; ++q) p[(size_t)q * npad] = acc[q];
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kWave) void k_grad_slice(const double* __restrict__
 // and stored as the sums of a single slice, so the sum pass reads NACC
 // values per particle instead of W * NACC and no partial sum of a slice
 // goes through HBM.
-template <bool SHEAR, bool BULK, int W, bool KEEP = false>
+template <bool SHEAR, bool BULK, int W, int FORM = kExact>
 __global__ __launch_bounds__(kWave * W) void k_grad_tile(const double* __restrict__ cand,
                                                          const int32_t* __restrict__ skey,
                                                          const int32_t* __restrict__ cell_off,
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kWave * W) void k_grad_tile(const double* __restric
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int slice = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // wave-uniform
   const int lane = threadIdx.x & (kWave - 1);
-  grad_walk<SHEAR, BULK, KEEP>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, m2h, tile, slice, W,
+  grad_walk<SHEAR, BULK, FORM>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, m2h, tile, slice, W,
                                [&](const double* acc) {
     #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -188,11 +188,11 @@ __global__ __launch_bounds__(256) void k_grad_sum(const double* __restrict__ can
 
 int launch_grad_pairs(ccake_event* ev)
 {
-  if (ev->p.pair_precision == 1) return launch_grad_pairs32(ev);
   const int n = ev->n_live;          // sorted positions of the live events' particles
   const double h = ev->p.hT;
   const double rc = 2.0 * h;
-  const double hinv2 = 1.0 / (h * h), m4h = -0.25 / h, m2h = -0.5 / h;
+  const bool single = ev->p.pair_precision == 1;
+  const double hinv2 = 1.0 / (h * h), m4h = (single ? -0.5 : -0.25) / h, m2h = (single ? -1.0 : -0.5) / h;
   const int ntiles = (n + kTile - 1) / kTile;
   const double rcs = search_radius(ev);
   const int W = grad_tile_waves(lds_slices(ev), ntiles, ev->dev->simds);
@@ -203,16 +203,20 @@ int launch_grad_pairs(ccake_event* ev)
       hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kWave * nw), 0, ev->stream, ev->cand_g, ev->skey, ev->cell_off,
                          ev->grid, n, rc * rc, rcs, hinv2, m4h, m2h, ev->part, ev->npad);
     };
-    auto waves = [&](auto w, auto keep) {
-      constexpr int V = decltype(w)::value;
-      constexpr bool K = decltype(keep)::value;
+    auto form = [&](auto w, auto f) {
+      constexpr int V = decltype(w)::value, FM = decltype(f)::value;
       const bool sh = ev->p.using_shear, bu = !ev->no_bulk;
-      if (sh) { if (bu) go(k_grad_tile<true, true, V, K>, V); else go(k_grad_tile<true, false, V, K>, V); }
-      else { if (bu) go(k_grad_tile<false, true, V, K>, V); else go(k_grad_tile<false, false, V, K>, V); }
+      if (sh) { if (bu) go(k_grad_tile<true, true, V, FM>, V); else go(k_grad_tile<true, false, V, FM>, V); }
+      else { if (bu) go(k_grad_tile<false, true, V, FM>, V); else go(k_grad_tile<false, false, V, FM>, V); }
     };
-    if (W >= 2 * kKeepGradWaves && keep_order(ev, ntiles)) waves(std::integral_constant<int, kKeepGradWaves>(), std::true_type());
-    else if (W == 8) waves(std::integral_constant<int, 8>(), std::false_type());
-    else waves(std::integral_constant<int, 4>(), std::false_type());
+    const std::integral_constant<int, 8> w8;
+    const std::integral_constant<int, 4> w4;
+    if (single && W == 8) form(w8, std::integral_constant<int, kSingle>());
+    else if (single) form(w4, std::integral_constant<int, kSingle>());
+    else if (W >= 2 * kKeepGradWaves && keep_order(ev, ntiles))
+      form(std::integral_constant<int, kKeepGradWaves>(), std::integral_constant<int, kKeep>());
+    else if (W == 8) form(w8, std::integral_constant<int, kExact>());
+    else form(w4, std::integral_constant<int, kExact>());
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
   }
   ev->grad_sum_slices = ev->nslices;
@@ -221,11 +225,13 @@ int launch_grad_pairs(ccake_event* ev)
     hipLaunchKernelGGL(kern, grid, blk, 0, ev->stream, ev->cand_g, ev->skey, ev->cell_off, ev->grid, n, rc * rc,
                        rcs, hinv2, m4h, m2h, ev->nslices, ev->part, ev->npad);
   };
-  if (ev->p.using_shear) {
-    if (ev->no_bulk) go(k_grad_slice<true, false>); else go(k_grad_slice<true, true>);
-  } else {
-    if (ev->no_bulk) go(k_grad_slice<false, false>); else go(k_grad_slice<false, true>);
-  }
+  auto form = [&](auto f) {
+    constexpr int FM = decltype(f)::value;
+    const bool bu = !ev->no_bulk;
+    if (ev->p.using_shear) { if (bu) go(k_grad_slice<true, true, FM>); else go(k_grad_slice<true, false, FM>); }
+    else { if (bu) go(k_grad_slice<false, true, FM>); else go(k_grad_slice<false, false, FM>); }
+  };
+  if (single) form(std::integral_constant<int, kSingle>()); else form(std::integral_constant<int, kExact>());
   return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
 }
 

@@ -4,6 +4,7 @@
 // the same walk counts neighbours (btrack, src/system_state.cpp:712-715)
 // and exports the pair set for parity checks.
 #include "pair_common.h"
+#include <type_traits>
 #include <vector>
 #include <algorithm>
 
@@ -185,12 +186,11 @@ template <int MODE>
 constexpr int smooth_nacc() { return (MODE == 0 || MODE == 3) ? 6 : 2; }
 
 // The walk of one (tile, slice) unit (one wave); fin(acc) receives the
-// slice's sums (sigma_lab, the pair count, then s, B, S, Q).  KEEP: with the
-// arithmetic of q_and_inverse and spline_w (keep_order).
+// slice's sums (sigma_lab, the pair count, then s, B, S, Q).
 // Bound: the FP64 vector unit, 23 instructions per candidate and wave in
 // MODE 0.  188,250 particles (479M pairs): 745 us per launch with 31
 // instructions and no request ahead, 610 us now.
-template <int MODE, bool KEEP, class Fin>
+template <int MODE, int FORM, class Fin>
 __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, const int32_t* __restrict__ skey,
                                             const int32_t* __restrict__ cell_off, const Grid* __restrict__ gridp,
                                             int n, double rc2, double rcs, double hinv2, double m4h, double mk2h, int tile, int slice,
@@ -211,19 +211,19 @@ __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, con
   for_segments(act, myrow, xi, yi, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
     const double xs = in ? xi : kFarAway;      // lanes of other cell rows sit this segment's walk out
-    for_spans_slice<kCandS, KEEP>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
+    for_spans_slice<kCandS, FORM == kKeep>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
       // whole records or half records: one scalar load each
       constexpr int NR = (MODE == 0) ? 8 : 4;
       walk_records<NR, kCandS, 1>(cand, xs, yi, cur,
                                [&](const double* c, double dx, double dy, double r2) {
         cnt += r2 <= rc2 ? 1 : 0;
         double w;
-        if (KEEP) {
+        if (FORM == kKeep) {
           double q, iq;
           q_and_inverse(r2, hinv2, q, iq);
           w = spline_w(q);
         } else {
-          w = spline_w8(r2, m4h, mk2h);
+          w = spline_w8<FORM>(r2, m4h, mk2h);
         }
         sl += c[2] * w;
         if (MODE == 0 || MODE == 3) ss += c[MODE == 1 ? 0 : 3] * w;
@@ -234,12 +234,12 @@ __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, con
       });
     });
   });
-  const double f = KEEP ? 1.0 : kSplineW;
+  const double f = FORM == kKeep ? 1.0 : kSplineW;
   const double acc[6] = { f * sl, (double)cnt, f * ss, f * sB, f * sS, f * sQ };
   fin(acc);
 }
 
-template <int MODE>
+template <int MODE, int FORM = kExact>
 __global__ __launch_bounds__(kWave) void k_smooth_slice(const double* __restrict__ cand,
                                                         const int32_t* __restrict__ skey,
                                                         const int32_t* __restrict__ cell_off,
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(kWave) void k_smooth_slice(const double* __restrict
   const int unit = xcd_tile(blockIdx.x, gridDim.x);
   const int tile = unit / nslices;
   const int slice = unit - tile * nslices;
-  smooth_walk<MODE, false>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, mk2h, tile, slice, nslices, [&](const double* acc) {
+  smooth_walk<MODE, FORM>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, mk2h, tile, slice, nslices, [&](const double* acc) {
     double* p = part + (size_t)slice * NACC * npad + tile * kTile + threadIdx.x;
     #pragma unroll
     for (int q = 0; q < NACC; ++q) p[(size_t)q * npad] = acc[q];
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(kWave) void k_smooth_slice(const double* __restrict
 
 // The W slices of a tile in one workgroup of W waves, their sums added in
 // slice order in LDS and stored as one slice's (as k_grad_tile).
-template <int MODE, int W, bool KEEP = false>
+template <int MODE, int W, int FORM = kExact>
 __global__ __launch_bounds__(kWave * W) void k_smooth_tile(const double* __restrict__ cand,
                                                            const int32_t* __restrict__ skey,
                                                            const int32_t* __restrict__ cell_off,
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(kWave * W) void k_smooth_tile(const double* __restr
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int slice = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // wave-uniform
   const int lane = threadIdx.x & (kWave - 1);
-  smooth_walk<MODE, KEEP>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, mk2h, tile, slice, W, [&](const double* acc) {
+  smooth_walk<MODE, FORM>(cand, skey, cell_off, gridp, n, rc2, rcs, hinv2, m4h, mk2h, tile, slice, W, [&](const double* acc) {
     #pragma unroll
     for (int q = 0; q < NACC; ++q) red[slice][q][lane] = acc[q];
   });
@@ -386,37 +386,43 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
                        ev->perm, ev->cell_off, ev->grid, n, rc2, rcs, bt, pc);
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
   }
-  if (mode == 0 && ev->p.pair_precision == 1) return launch_smooth_pairs32(ev);
-  const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT), m4h = -0.25 / ev->p.hT, mk2h = -0.5 * kSplineK / ev->p.hT;
   const int W = lds_slices(ev);
+  const int m = (mode == 0 && ev->no_charges) ? 3 : mode;
+  // the initial sigma stays in FP64 with pair_precision 1
+  const bool single = mode == 0 && ev->p.pair_precision == 1;
+  const bool keep = !single && W >= kKeepSmoothWaves && keep_order(ev, ntiles);
+  const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT), m4h = (single ? -0.5 : -0.25) / ev->p.hT;
+  const double mk2h = (single ? -1.0 : -0.5) * kSplineK / ev->p.hT;
   if (W) {
     // the tile's slices reduced in LDS: the sum pass sees one slice
     ev->smooth_sum_slices = 1;
-    auto launch = [&](auto kern, int waves) {
+    auto go = [&](auto kern, int waves) {
       hipLaunchKernelGGL(kern, dim3(ntiles), dim3(kWave * waves), 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n,
                          rc2, rcs, hinv2, m4h, mk2h, ev->part, ev->npad);
     };
-    auto go = [&](auto kern) { launch(kern, W); };
-    const int m = (mode == 0 && ev->no_charges) ? 3 : mode;
-    if (W >= kKeepSmoothWaves && keep_order(ev, ntiles)) {
-      if (m == 3) launch(k_smooth_tile<3, kKeepSmoothWaves, true>, kKeepSmoothWaves);
-      else if (m == 0) launch(k_smooth_tile<0, kKeepSmoothWaves, true>, kKeepSmoothWaves);
-      else launch(k_smooth_tile<1, kKeepSmoothWaves, true>, kKeepSmoothWaves);
-    } else if (W == 8) { if (m == 3) go(k_smooth_tile<3, 8>); else if (m == 0) go(k_smooth_tile<0, 8>); else go(k_smooth_tile<1, 8>); }
-    else { if (m == 3) go(k_smooth_tile<3, 4>); else if (m == 0) go(k_smooth_tile<0, 4>); else go(k_smooth_tile<1, 4>); }
+    auto form = [&](auto w, auto f) {
+      constexpr int V = decltype(w)::value, FM = decltype(f)::value;
+      if (m == 3) go(k_smooth_tile<3, V, FM>, V);
+      else if (m == 0) go(k_smooth_tile<0, V, FM>, V);
+      else if constexpr (FM != kSingle) go(k_smooth_tile<1, V, FM>, V);
+    };
+    const std::integral_constant<int, 8> w8;
+    const std::integral_constant<int, 4> w4;
+    if (keep) form(std::integral_constant<int, kKeepSmoothWaves>(), std::integral_constant<int, kKeep>());
+    else if (single && W == 8) form(w8, std::integral_constant<int, kSingle>());
+    else if (single) form(w4, std::integral_constant<int, kSingle>());
+    else if (W == 8) form(w8, std::integral_constant<int, kExact>());
+    else form(w4, std::integral_constant<int, kExact>());
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
   }
   ev->smooth_sum_slices = ev->nslices;
-  const dim3 grid(ntiles * ev->nslices), blk(kWave);
-  if (mode == 0 && ev->no_charges)
-    hipLaunchKernelGGL(k_smooth_slice<3>, grid, blk, 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n, rc2,
-                       rcs, hinv2, m4h, mk2h, ev->nslices, ev->part, ev->npad);
-  else if (mode == 0)
-    hipLaunchKernelGGL(k_smooth_slice<0>, grid, blk, 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n, rc2,
-                       rcs, hinv2, m4h, mk2h, ev->nslices, ev->part, ev->npad);
-  else
-    hipLaunchKernelGGL(k_smooth_slice<1>, grid, blk, 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid, n, rc2,
-                       rcs, hinv2, m4h, mk2h, ev->nslices, ev->part, ev->npad);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(ntiles * ev->nslices), dim3(kWave), 0, st, ev->cand_s, ev->skey, ev->cell_off, ev->grid,
+                       n, rc2, rcs, hinv2, m4h, mk2h, ev->nslices, ev->part, ev->npad);
+  };
+  if (m == 3) { if (single) go(k_smooth_slice<3, kSingle>); else go(k_smooth_slice<3>); }
+  else if (m == 0) { if (single) go(k_smooth_slice<0, kSingle>); else go(k_smooth_slice<0>); }
+  else go(k_smooth_slice<1>);
   return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
 }
 

@@ -183,31 +183,6 @@ __device__ __forceinline__ void row_run(const Grid& g, const int32_t* __restrict
   e = cell_off[kr + cx1 + 1];
 }
 
-// Skip a candidate (wave-uniform branch) when it is out of range for every
-// active lane: such candidates lie in the cell-rounding margin of the
-// tile's region, and every lane would add exact zeros.  On by default
-// (measured 10 % faster at 40k particles); the records are requested before
-// the branch, so it does not hold up the loads.
-#ifndef CCAKE_PAIR_SKIP
-#define CCAKE_PAIR_SKIP 1
-#endif
-constexpr bool kSkipEmpty = CCAKE_PAIR_SKIP != 0;
-
-// The skip test: no lane of the wave has `p` set.  It runs inside the walk's
-// body, on the lanes of one segment.  The host emulation build (kernels
-// compiled for the CPU to check memory accesses) runs every candidate
-// instead, since its lanes do not execute the body in lockstep; the records
-// are read before the test either way, so the accesses are the same.
-__device__ __forceinline__ bool wave_none(bool p)
-{
-#ifdef CCAKE_HOST_EMU
-  (void)p;
-  return false;
-#else
-  return __ballot(p) == 0ull;
-#endif
-}
-
 // The candidates of one slice of a segment that can be in range, in order,
 // 64 cell rows' worth (the rows are resolved lane-parallel, lane r holding
 // row r's run, so their cell offsets arrive with one vector load).  The
@@ -516,30 +491,47 @@ __device__ __forceinline__ double spline_g(double q, double iq)
 constexpr double kFarAway = 1e100;
 constexpr double kSplineW = 8.0;                     // spline_w / spline_w8
 __device__ __forceinline__ double clamp01(double v) { return fmin(fmax(v, 0.0), 1.0); }
-// 2 r of a pair; ir2 receives 2 / r
+// FORM of a walk: kExact with the arithmetic above; kKeep with that of
+// q_and_inverse, spline_w and spline_g (keep_order); kSingle without the
+// Newton step (pair_precision 1): y and f as they are, so r and 1/r instead of
+// 2 r and 2 / r, with v_rsq_f64's relative error (5.2e-8 at most, 1.0e-8
+// rms over 4M arguments: less than one rounding to single precision),
+// everything else in FP64.  Single-precision arithmetic would not be faster: it
+// issues at the FP64 rate here.  188,250 particles: smoothing 615 -> 583 us,
+// gradients 968 -> 915 us (pair terms in FP32 with compensated sums: 557 and 986).  The constants m4h
+// and m2h (mk2h) are then twice as large, and the gradient's final factor.
+enum Form { kExact, kKeep, kSingle };
+// 2 r of a pair; ir2 receives 2 / r (kSingle: r and 1 / r)
+template <int FORM>
 __device__ __forceinline__ double twice_r(double r2, double& ir2)
 {
   const double x = r2 + 1e-300;
   const double y = __builtin_amdgcn_rsq(x);
   const double f = x * y;
+  if (FORM == kSingle) {
+    ir2 = y;
+    return f;
+  }
   const double e = fma(-f, y, 3.0);
   ir2 = y * e;
   return f * e;
 }
-// (t^2 - u^2) * 2 / r; m4h = -1 / (4 h), m2h = -1 / (2 h)
+// (t^2 - u^2) * 2 / r; m4h = -1 / (4 h), m2h = -1 / (2 h) (kSingle: twice those, and half the result)
+template <int FORM = kExact>
 __device__ __forceinline__ double spline_g2(double r2, double m4h, double m2h)
 {
   double ir2;
-  const double d = twice_r(r2, ir2);
+  const double d = twice_r<FORM>(r2, ir2);
   const double t = clamp01(fma(d, m4h, 1.0)), u = clamp01(fma(d, m2h, 1.0));
   return fma(-u, u, t * t) * ir2;
 }
 // t^3 - (k u)^3
 constexpr double kSplineK = 0.79370052598409973738;  // 2^(-1/3)
+template <int FORM = kExact>
 __device__ __forceinline__ double spline_w8(double r2, double m4h, double mk2h)
 {
   double ir2;
-  const double d = twice_r(r2, ir2);
+  const double d = twice_r<FORM>(r2, ir2);
   const double t = clamp01(fma(d, m4h, 1.0)), u = clamp01(fma(d, mk2h, kSplineK));
   return fma(-(u * u), u, (t * t) * t);
 }

@@ -176,10 +176,12 @@ typedef struct ccake_params {
   /* Precision of the time step's smoothing and gradient pair sums (no
      counterpart in the reference, which is FP64 throughout):
      0 FP64 (the reference's arithmetic);
-     1 FP32 pair terms with compensated FP32 accumulation.  Positions, the
-       pair predicate (so the pair set), the slices' sums and everything
+     1 single-precision pair weights: the kernel's r and 1/r from the
+       hardware reciprocal square root alone (relative error 5.2e-8 at most),
+       without the step that refines it to FP64.  Positions, the pair
+       predicate (so the pair set), the products and sums and everything
        outside the pair loops (EoS inversion, EoM, RK accumulation, shear
-       update, initialisation, diffusion sums) stay FP64. */
+       update, initialisation, diffusion sums) are FP64. */
   int    pair_precision;
   /* D = 3 only: the factorized kernel W_2D(r_perp, hT) W_1D(|d eta|, hEta)
      (SPHkernel<3>::kernel / gradKernel, src/kernel.cpp:129-170; selected by

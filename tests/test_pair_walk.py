@@ -94,3 +94,30 @@ def test_sort_and_counts(dev, n):
     assert np.array_equal(ev.download_int("CCAKE_I_BTRACK"), want)
     ev.close()
     eos.close()
+
+
+# single-precision weights (relative error 5.2e-8 at most) with each number of
+# waves per tile and with single-wave slices: a smoothed field is a sum of
+# positive terms, so its error stays below that; the gradients cancel
+@pytest.mark.parametrize("slices", [8, 4, 2])
+@pytest.mark.parametrize("shear", [0, 1])
+def test_single_precision_weights(dev, slices, shear):
+    d = cloud(2500, 2.5)
+    cfg = config.base_params(t0=0.6, dt=0.01, particlization=0, eta_mode=config.ETA_CONSTANT,
+                             constant_eta_over_s=0.08 if shear else 0.0, cells_per_rc=4, x_subcells=4)
+    eos = ccake_amd.Eos(dev, 0, 0.75)
+    got = []
+    for pp in (0, 1):
+        ev = ccake_amd.Event(dev, eos, dict(cfg, pair_precision=pp), len(d["x"]))
+        ccake_amd.load_event(ev, d)
+        ev.nslices(slices)
+        ev.initialize()
+        ev.get_time_derivatives()
+        got.append({f: ev.download(ccake_amd.FIELDS["CCAKE_F_" + f]) for f in ("SIGMA_LAB", "S", "GRADP0", "GRADE0", "GRADV0")})
+        got[-1]["BTRACK"] = ev.download_int("CCAKE_I_BTRACK")
+        ev.close()
+    eos.close()
+    assert np.array_equal(got[0].pop("BTRACK"), got[1].pop("BTRACK"))
+    for f, a in got[0].items():
+        err = np.max(np.abs(got[1][f] - a)) / np.max(np.abs(a))
+        assert 0.0 < err <= (5.2e-8 if f == "SIGMA_LAB" else 2e-6), (f, err)
