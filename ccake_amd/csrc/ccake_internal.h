@@ -180,7 +180,8 @@ struct ccake_event {
   int init_phase = 0;               // initialisation phases done (1, 2, 3)
   // pair-kernel partial sums: nslices x (up to 17) x npad, sorted order
   int nslices = 1;
-  int nslices_cap = 1;          // slices the partial-sum buffer holds
+  int nslices_cap = 1;          // largest slice count the event accepts
+  int part_slices = 1;          // slices the partial-sum buffer holds
   // EoS stage: particles whose inversion needs the full cascade (positions),
   // two alternating counters and which one the next stage appends to
   double* k4 = nullptr;         // RK4 accumulator (allocated at the first fourth-order step)

@@ -219,13 +219,13 @@ int launch_diff_prep(ccake_event* ev, int what, const int32_t* perm)
 }
 
 template <int S = 1>
-static int diff_sum_dispatch(ccake_event* ev, double C)
+static int diff_sum_dispatch(ccake_event* ev, int slices, double C)
 {
   if constexpr (S > kMaxSlices) {
     set_error("slice count out of range");
     return CCAKE_ERR_INVALID;
   } else {
-    if (ev->nslices != S) return diff_sum_dispatch<S + 1>(ev, C);
+    if (slices != S) return diff_sum_dispatch<S + 1>(ev, slices, C);
     const int n = ev->n_live;
     hipLaunchKernelGGL((k_diff_sum<S>), dim3((n + 255) / 256), dim3(256), 0, ev->stream, ev->cand_d, ev->perm, n, C,
                        ev->part, ev->npad, ev->F);
@@ -239,12 +239,13 @@ int launch_diff_grad(ccake_event* ev)
   const double h = ev->p.hT;
   const double rc = 2.0 * h;
   const int ntiles = (n + kTile - 1) / kTile;
-  hipLaunchKernelGGL(k_diff_slice, dim3(ntiles * ev->nslices), dim3(kWave), 0, ev->stream, ev->cand_d, ev->skey,
-                     ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), -0.25 / h, -0.5 / h, ev->nslices, ev->part,
+  const int slices = ev->nslices < ev->part_slices ? ev->nslices : ev->part_slices;   // each slice's sums are stored
+  hipLaunchKernelGGL(k_diff_slice, dim3(ntiles * slices), dim3(kWave), 0, ev->stream, ev->cand_d, ev->skey,
+                     ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), -0.25 / h, -0.5 / h, slices, ev->part,
                      ev->npad);
   if (hipGetLastError() != hipSuccess) return CCAKE_ERR_HIP;
   const double C = -0.5 * (15.0 / (7.0 * kPi)) / pow(h, 4);
-  const int rc2 = diff_sum_dispatch(ev, C);
+  const int rc2 = diff_sum_dispatch(ev, slices, C);
   if (rc2) return rc2;
   return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;
 }

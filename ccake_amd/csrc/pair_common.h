@@ -1,10 +1,10 @@
-// Shared device helpers of the pair kernels (smoothing, gradients, pair
-// export).  A workgroup is one wave; its 64 lanes own 64 consecutive
-// particles of the cell-sorted order (a "tile").  The tile's bounding box
-// selects, row by row, the contiguous run of cells within the interaction
-// radius; every lane then walks that run in the same order, so the
-// candidate index is wave-uniform and candidate records are fetched with
-// scalar loads into SGPRs instead of being staged through LDS.
+// Shared device helpers of the pair kernels (smoothing, gradients,
+// diffusion, neighbour counts, pair export).  A wave's 64 lanes own 64
+// consecutive particles of the cell-sorted order (a "tile").  The tile's
+// bounding box selects, row by row, the contiguous run of cells within the
+// interaction radius; every lane then walks the candidates in the same order,
+// so the candidate index is wave-uniform and candidate records are fetched
+// with scalar loads into SGPRs instead of being staged through LDS.
 #pragma once
 #include "ccake_internal.h"
 #include <climits>
@@ -159,10 +159,10 @@ __device__ __forceinline__ int xcd_tile(int bid, int nblk)
 }
 
 // Hot pair kernels split a tile's flattened candidate list into `nslices`
-// contiguous slices; slice `slice` is walked by one wave (one workgroup), so
-// the work units are small enough to spread evenly over the chip's SIMDs
-// even when there are few tiles.  Every wave of a tile computes the same
-// segments and spans (wave-uniform values).
+// slices, each walked by one wave (the waves of one workgroup, or workgroups
+// of one wave), so the work units are small enough to spread evenly over the
+// chip's SIMDs even when there are few tiles.  Every wave of a tile computes
+// the same segments and spans (wave-uniform values).
 
 // Candidate run of cell row ry0 + r for a segment: [b, e) in sorted order
 // (empty when r >= nrow or the row is out of reach).  Evaluated per lane.
@@ -304,7 +304,8 @@ __device__ __forceinline__ void for_spans_slice(const Grid& g, const int32_t* __
 
 // Number of slices per tile for `ntiles` tiles on `simds` SIMDs: the
 // smallest that gives near-whole rounds of single-wave work units and at
-// least about four waves per SIMD (to hide load latency), at most 16.
+// least about four waves per SIMD (to hide load latency), at most 16.  It sets
+// how many slices an event accepts (ccake_event_pair_slices).
 inline int choose_slices(int ntiles, int simds)
 {
   int best = 1;

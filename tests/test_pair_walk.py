@@ -121,3 +121,35 @@ def test_single_precision_weights(dev, slices, shear):
     for f, a in got[0].items():
         err = np.max(np.abs(got[1][f] - a)) / np.max(np.abs(a))
         assert 0.0 < err <= (5.2e-8 if f == "SIGMA_LAB" else 2e-6), (f, err)
+
+
+# An event for which one slice of partial sums is set aside (262,144 particles
+# are 4,096 tiles: whole rounds of the chip's SIMDs) runs its tiles of 8 waves in
+# no more device memory: the diffusion pass, which stores every slice's sums,
+# then takes one slice, and a slice count whose sums would not fit is refused.
+def test_partial_sums_fit(dev):
+    n = 262144
+    m = 512
+    x, y = (a.ravel() for a in np.meshgrid(np.arange(m) * 0.1, np.arange(m) * 0.1))
+    cfg = config.base_params(t0=0.6, dt=0.01, particlization=0, cells_per_rc=4, x_subcells=4, using_diffusion=1,
+                             kappa_over_T2=[0.1, 0, 0, 0, 0.1, 0, 0, 0, 0.1], diffusion_regulator=1)
+    f = 0.02 * np.cos(x + 0.3 * y)
+    e = 10.0 + np.cos(0.1 * x) + np.cos(0.1 * y)
+    d = dict(x=x, y=y, e=e, ux=0.05 * np.sin(0.2 * x), uy=0.05 * np.sin(0.3 * y), rhoB=f * e, rhoS=0.5 * f * e, rhoQ=-f * e)
+    eos = ccake_amd.Eos(dev, 0, 0.75)
+    ev = ccake_amd.Event(dev, eos, cfg, n)
+    ccake_amd.load_event(ev, d)
+    assert ev.nslices() == 8
+    ev.initialize()
+    ev.get_time_derivatives()
+    a = [ev.download(ccake_amd.FIELDS["CCAKE_F_" + f]) for f in ("GRADP0", "GRADV0", "DEXT_Q0")]
+    ev.nslices(4)
+    for s in (2, 3, 16):
+        with pytest.raises(RuntimeError):
+            ev.nslices(s)
+    ev.nslices(1)
+    ev.get_time_derivatives()
+    for u, v in zip(a, (ev.download(ccake_amd.FIELDS["CCAKE_F_" + f]) for f in ("GRADP0", "GRADV0", "DEXT_Q0"))):
+        assert np.max(np.abs(u - v)) <= 1e-12 * np.max(np.abs(u)) > 0.0
+    ev.close()
+    eos.close()
