@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kWave) void k_diff_slice(const double* __restrict__
   double acc[kDiffAcc];
   for (int q = 0; q < kDiffAcc; ++q) acc[q] = 0.0;
 
-  for_segments(act, myrow, xa, ya, [&](const Seg& seg, bool in) {
+  for_segments(gridp, g0, 0.0, act, myrow, xa, ya, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
     const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
     for_spans_slice<kCandD, false>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {

@@ -54,7 +54,7 @@ __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const
   #pragma unroll
   for (int q = 0; q < NW; ++q) acc[q] = 0.0;
 
-  for_segments(act, myrow, xa, ya, [&](const Seg& seg, bool in) {
+  for_segments(gridp, g0, FORM == kSmall ? rcs : 0.0, act, myrow, xa, ya, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
     const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
     for_spans_slice<kCandG, KEEP>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
@@ -215,6 +215,7 @@ int launch_grad_pairs(ccake_event* ev)
     else if (single) form(w4, std::integral_constant<int, kSingle>());
     else if (W >= 2 * kKeepGradWaves && keep_order(ev, ntiles))
       form(std::integral_constant<int, kKeepGradWaves>(), std::integral_constant<int, kKeep>());
+    else if (W == 8 && small_event(ev, ntiles)) form(w8, std::integral_constant<int, kSmall>());
     else if (W == 8) form(w8, std::integral_constant<int, kExact>());
     else form(w4, std::integral_constant<int, kExact>());
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;

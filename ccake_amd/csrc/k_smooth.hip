@@ -110,7 +110,7 @@ __global__ __launch_bounds__(64) void k_export(const double* __restrict__ cand,
   const int id = act ? perm[kk] : 0;
   int64_t wpos = act ? row_off[id] : 0;
 
-  for_segments(act, myrow, xi, yi, [&](const Seg& seg, bool in) {
+  for_segments(gridp, g0, 0.0, act, myrow, xi, yi, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
     for_spans(g, cell_off, seg, rcs, [&](int j) {
       const double* c = cand + (size_t)j * kCandS;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kWave * W) void k_count_tile(const double* __restri
   const double xi = me[0], yi = me[1];
   const int myrow = act ? skey[kk] / g0.stride : INT_MAX;
   int cnt = 0;
-  for_segments(act, myrow, xi, yi, [&](const Seg& seg, bool in) {
+  for_segments(gridp, g0, 0.0, act, myrow, xi, yi, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
     const double xs = in ? xi : kFarAway;
     for_spans_slice<kCandS, false>(g, cell_off, cand, seg, rc2, rcs, slice, W, [&](RunCursor& cur) {
@@ -208,7 +208,7 @@ __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, con
   double sl = 0.0, ss = 0.0, sB = 0.0, sS = 0.0, sQ = 0.0;
   int cnt = 0;   // r2 <= rc2, the self pair included
 
-  for_segments(act, myrow, xi, yi, [&](const Seg& seg, bool in) {
+  for_segments(gridp, g0, FORM == kSmall ? rcs : 0.0, act, myrow, xi, yi, [&](const Seg& seg, bool in) {
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
     const double xs = in ? xi : kFarAway;      // lanes of other cell rows sit this segment's walk out
     for_spans_slice<kCandS, FORM == kKeep>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
@@ -411,6 +411,7 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
     if (keep) form(std::integral_constant<int, kKeepSmoothWaves>(), std::integral_constant<int, kKeep>());
     else if (single && W == 8) form(w8, std::integral_constant<int, kSingle>());
     else if (single) form(w4, std::integral_constant<int, kSingle>());
+    else if (W == 8 && small_event(ev, ntiles)) form(w8, std::integral_constant<int, kSmall>());
     else if (W == 8) form(w8, std::integral_constant<int, kExact>());
     else form(w4, std::integral_constant<int, kExact>());
     return hipGetLastError() == hipSuccess ? 0 : CCAKE_ERR_HIP;

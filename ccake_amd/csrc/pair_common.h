@@ -346,6 +346,8 @@ inline bool keep_order(const ccake_event* ev, int ntiles)
   return ev->snaps && 8 * ntiles <= ev->dev->simds;
 }
 constexpr int kKeepSmoothWaves = 8, kKeepGradWaves = 4;
+// An event (or batch) of at most a wave per SIMD (for_segments).
+inline bool small_event(const ccake_event* ev, int ntiles) { return 8 * ntiles <= ev->dev->simds; }
 
 // Per-slice partial sums: part[(slice * nacc + f) * npad + k] for sorted
 // position k (every tile lane, k < ntiles * 64 <= npad, has a slot).
@@ -501,7 +503,9 @@ __device__ __forceinline__ double clamp01(double v) { return fmin(fmax(v, 0.0), 
 // issues at the FP64 rate here.  188,250 particles: smoothing 615 -> 583 us,
 // gradients 968 -> 915 us (pair terms in FP32 with compensated sums: 557 and 986).  The constants m4h
 // and m2h (mk2h) are then twice as large, and the gradient's final factor.
-enum Form { kExact, kKeep, kSingle };
+// kSmall: kExact with the rows of a tile as one segment where that reaches less
+// (for_segments), for events whose waves do not fill the SIMDs.
+enum Form { kExact, kKeep, kSingle, kSmall };
 // 2 r of a pair; ir2 receives 2 / r (kSingle: r and 1 / r)
 template <int FORM>
 __device__ __forceinline__ double twice_r(double r2, double& ir2)
@@ -537,22 +541,56 @@ __device__ __forceinline__ double spline_w8(double r2, double m4h, double mk2h)
   return fma(-(u * u), u, (t * t) * t);
 }
 
+// The lanes' bounding box (wave-uniform).
+__device__ __forceinline__ Seg box_of(int row, bool in, double xi, double yi)
+{
+  Seg s;
+  s.row = row;
+  s.xmn = wave_min_d(in ? xi : INFINITY);
+  s.xmx = wave_max_d(in ? xi : -INFINITY);
+  s.ymn = wave_min_d(in ? yi : INFINITY);
+  s.ymx = wave_max_d(in ? yi : -INFINITY);
+  return s;
+}
+
 // Iterate over the row segments of the tile owned by this wave.  `fn(seg,
 // in_seg)` runs once per segment with in_seg true on the lanes of the segment.
 // Sorted positions have ascending key rows, so a segment is a run of lanes.
+// With rc > 0 (kSmall) the rows of a tile are one segment where that reaches less: when
+// the area within rc of the tile's box is smaller than the rows' areas
+// together (a tile of short rows, which its rows' walks would cover row by row
+// with some of the lanes each).  A tile of two long rows is the end of one and
+// the start of the next, far apart, and stays two segments, as do the rows of
+// two events.  2,601 particles in rows of 51: smoothing 25 -> 18 us, gradients
+// 28 -> 20; 30,300 in rows of 174, where few tiles hold more than two: 50 -> 52
+// and 69 -> 71, for the boxes.  So only while 8 waves a tile fill no more than
+// the SIMDs (small_event).
 template <class Fn>
-__device__ __forceinline__ void for_segments(bool act, int myrow, double xi, double yi, Fn&& fn)
+__device__ __forceinline__ void for_segments(const Grid* __restrict__ gp, const Grid& g0, double rc, bool act, int myrow,
+                                             double xi, double yi, Fn&& fn)
 {
   uint64_t todo = __ballot(act);
+  bool whole = false;
+  if (rc > 0.0 && todo) {
+    const int l0 = __builtin_ctzll(todo), l1 = kWave - 1 - __builtin_clzll(todo);
+    const int first = __builtin_amdgcn_readlane(myrow, l0), last = __builtin_amdgcn_readlane(myrow, l1);
+    if (first != last && event_index(gp, g0, first) == event_index(gp, g0, last)) {
+      double apart = 0.0;
+      for (uint64_t t = todo; t;) {
+        const int r = __builtin_amdgcn_readlane(myrow, __builtin_ctzll(t));
+        const bool in = act && myrow == r;
+        const Seg s = box_of(r, in, xi, yi);
+        apart += (s.xmx - s.xmn + 2.0 * rc) * (s.ymx - s.ymn + 2.0 * rc);
+        t &= ~__ballot(in);
+      }
+      const Seg s = box_of(first, act, xi, yi);
+      whole = (s.xmx - s.xmn + 2.0 * rc) * (s.ymx - s.ymn + 2.0 * rc) < apart;
+    }
+  }
   while (todo) {
     const int r = __builtin_amdgcn_readlane(myrow, __builtin_ctzll(todo));
-    const bool in = act && myrow == r;
-    Seg s;
-    s.row = r;
-    s.xmn = wave_min_d(in ? xi : INFINITY);
-    s.xmx = wave_max_d(in ? xi : -INFINITY);
-    s.ymn = wave_min_d(in ? yi : INFINITY);
-    s.ymx = wave_max_d(in ? yi : -INFINITY);
+    const bool in = act && (whole || myrow == r);
+    const Seg s = box_of(r, in, xi, yi);
     fn(s, in);
     todo &= ~__ballot(in);
   }
