@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kWave) void k_diff_slice(const double* __restrict__
                                                       double rc2, double rcs, double m4h, double m2h, int nslices,
                                                       double* __restrict__ part, int npad)
 {
-  const Grid g0 = *gridp;
+  const Grid& g0 = *gridp;
   const int lane = threadIdx.x;
   const int unit = xcd_tile(blockIdx.x, gridDim.x);
   const int tile = unit / nslices;
@@ -134,29 +134,30 @@ __global__ __launch_bounds__(kWave) void k_diff_slice(const double* __restrict__
   const int myrow = act ? skey[kk] / g0.stride : INT_MAX;
 
   double acc[kDiffAcc];
-  for (int q = 0; q < kDiffAcc; ++q) acc[q] = 0.0;
-
-  for_segments(gridp, g0, 0.0, act, myrow, xa, ya, [&](const Seg& seg, bool in) {
-    const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
-    for_spans_slice<kCandD, false>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
-      walk_records<15, kCandD, 1>(cand, xs, ya, cur,
-                               [&](const double* c, double dx, double dy, double r2) {
-        const double gm = c[2] * spline_g2(r2, m4h, m2h);
-        const double wx = gm * dx, wy = gm * dy;
-        acc[0] += wx; acc[1] += wy;
-        #pragma unroll
-        for (int ch = 0; ch < 3; ++ch) {
-          acc[2 + ch] += c[3 + ch] * wx; acc[5 + ch] += c[3 + ch] * wy;      // q0_b / sl_b^2
-          acc[8 + ch] += c[6 + ch] * wx + c[9 + ch] * wy;                    // q^i_b / sl_b^2
-          acc[11 + ch] += c[12 + ch] * wx; acc[14 + ch] += c[12 + ch] * wy;  // alpha_b
-        }
+  for_tile_sums<kDiffAcc>(acc, [&](auto in_range) {
+    for_segments(gridp, g0, 0.0, act, myrow, xa, ya, [&](const Seg& seg, bool in) {
+      const Grid& g = gridp[event_index(gridp, g0, seg.row)];
+      const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
+      for_spans_slice<kCandD, false>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
+        walk_records<15, kCandD, decltype(in_range)::value>(cand, xs, ya, rc2, cur,
+                                 [&](const double* c, double dx, double dy, double r2) {
+          const double gm = c[2] * spline_g2(r2, m4h, m2h);
+          const double wx = gm * dx, wy = gm * dy;
+          acc[0] += wx; acc[1] += wy;
+          #pragma unroll
+          for (int ch = 0; ch < 3; ++ch) {
+            acc[2 + ch] += c[3 + ch] * wx; acc[5 + ch] += c[3 + ch] * wy;      // q0_b / sl_b^2
+            acc[8 + ch] += c[6 + ch] * wx; acc[8 + ch] += c[9 + ch] * wy;         // q^i_b / sl_b^2
+            acc[11 + ch] += c[12 + ch] * wx; acc[14 + ch] += c[12 + ch] * wy;  // alpha_b
+          }
+        });
       });
     });
   });
 
   const double h2 = -1.0 / m2h;                // spline_g2's factor
   double* p = part + (size_t)slice * kDiffAcc * npad + k;
+  #pragma unroll
   for (int q = 0; q < kDiffAcc; ++q) p[(size_t)q * npad] = h2 * acc[q];
 }
 

@@ -51,43 +51,42 @@ __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const
   constexpr int NW = SHEAR ? (KEEP ? 17 : 18) : 12;
   const double vax = me[6], vay = me[7];
   double acc[NW];
-  #pragma unroll
-  for (int q = 0; q < NW; ++q) acc[q] = 0.0;
-
-  for_segments(gridp, g0, FORM == kSmall ? rcs : 0.0, act, myrow, xa, ya, [&](const Seg& seg, bool in) {
-    const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
-    for_spans_slice<kCandG, KEEP>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
-      constexpr int NR = SHEAR ? 13 : 8;
-      walk_records<NR, kCandG, 1>(cand, xs, ya, cur,
-                               [&](const double* c, double dx, double dy, double r2) {
-        double gm;
-        if (KEEP) {
-          double q, iq;
-          q_and_inverse(r2, hinv2, q, iq);
-          gm = c[2] * spline_g(q, iq);
-        } else {
-          gm = c[2] * spline_g2<FORM>(r2, m4h, m2h);
-        }
-        const double wx = gm * dx, wy = gm * dy;
-        acc[0] += wx; acc[1] += wy;                    // sum m_b grad W
-        acc[2] += c[3] * wx; acc[3] += c[3] * wy;      // p_b / sl_b^2
-        acc[4] += c[4] * wx; acc[5] += c[4] * wy;      // e_b
-        if (BULK) { acc[6] += c[5] * wx; acc[7] += c[5] * wy; }   // Pi_b / sl_b^2
-        acc[8] += c[6] * wx; acc[9] += c[7] * wx;      // v_b d_x W
-        acc[10] += c[6] * wy; acc[11] += c[7] * wy;    // v_b d_y W
-        if (SHEAR && KEEP) {
-          const double cv = wx * vax + wy * vay;
-          acc[SHEAR ? 12 : 0] += cv;
-          acc[SHEAR ? 13 : 0] += cv * c[SHEAR ? 8 : 0]; acc[SHEAR ? 14 : 0] += cv * c[SHEAR ? 9 : 0];
-          acc[SHEAR ? 15 : 0] += wx * c[SHEAR ? 10 : 0] + wy * c[SHEAR ? 11 : 0];
-          acc[SHEAR ? 16 : 0] += wx * c[SHEAR ? 11 : 0] + wy * c[SHEAR ? 12 : 0];
-        } else if (SHEAR) {
-          acc[SHEAR ? 12 : 0] += c[SHEAR ? 8 : 0] * wx; acc[SHEAR ? 13 : 0] += c[SHEAR ? 8 : 0] * wy;
-          acc[SHEAR ? 14 : 0] += c[SHEAR ? 9 : 0] * wx; acc[SHEAR ? 15 : 0] += c[SHEAR ? 9 : 0] * wy;
-          acc[SHEAR ? 16 : 0] += c[SHEAR ? 10 : 0] * wx; acc[SHEAR ? 16 : 0] += c[SHEAR ? 11 : 0] * wy;
-          acc[NW - 1] += c[SHEAR ? 11 : 0] * wx; acc[NW - 1] += c[SHEAR ? 12 : 0] * wy;
-        }
+  for_tile_sums<NW>(acc, [&](auto in_range) {
+    for_segments(gridp, g0, FORM == kSmall ? rcs : 0.0, act, myrow, xa, ya, [&](const Seg& seg, bool in) {
+      const Grid& g = gridp[event_index(gridp, g0, seg.row)];
+      const double xs = in ? xa : kFarAway;      // lanes of other cell rows sit this segment's walk out
+      for_spans_slice<kCandG, KEEP>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
+        constexpr int NR = SHEAR ? 13 : 8;
+        walk_records<NR, kCandG, decltype(in_range)::value>(cand, xs, ya, rc2, cur,
+                                 [&](const double* c, double dx, double dy, double r2) {
+          double gm;
+          if (KEEP) {
+            double q, iq;
+            q_and_inverse(r2, hinv2, q, iq);
+            gm = c[2] * spline_g(q, iq);
+          } else {
+            gm = c[2] * spline_g2<FORM>(r2, m4h, m2h);
+          }
+          const double wx = gm * dx, wy = gm * dy;
+          acc[0] += wx; acc[1] += wy;                    // sum m_b grad W
+          acc[2] += c[3] * wx; acc[3] += c[3] * wy;      // p_b / sl_b^2
+          acc[4] += c[4] * wx; acc[5] += c[4] * wy;      // e_b
+          if (BULK) { acc[6] += c[5] * wx; acc[7] += c[5] * wy; }   // Pi_b / sl_b^2
+          acc[8] += c[6] * wx; acc[9] += c[7] * wx;      // v_b d_x W
+          acc[10] += c[6] * wy; acc[11] += c[7] * wy;    // v_b d_y W
+          if (SHEAR && KEEP) {
+            const double cv = wx * vax + wy * vay;
+            acc[SHEAR ? 12 : 0] += cv;
+            acc[SHEAR ? 13 : 0] += cv * c[SHEAR ? 8 : 0]; acc[SHEAR ? 14 : 0] += cv * c[SHEAR ? 9 : 0];
+            acc[SHEAR ? 15 : 0] += wx * c[SHEAR ? 10 : 0] + wy * c[SHEAR ? 11 : 0];
+            acc[SHEAR ? 16 : 0] += wx * c[SHEAR ? 11 : 0] + wy * c[SHEAR ? 12 : 0];
+          } else if (SHEAR) {
+            acc[SHEAR ? 12 : 0] += c[SHEAR ? 8 : 0] * wx; acc[SHEAR ? 13 : 0] += c[SHEAR ? 8 : 0] * wy;
+            acc[SHEAR ? 14 : 0] += c[SHEAR ? 9 : 0] * wx; acc[SHEAR ? 15 : 0] += c[SHEAR ? 9 : 0] * wy;
+            acc[SHEAR ? 16 : 0] += c[SHEAR ? 10 : 0] * wx; acc[SHEAR ? 16 : 0] += c[SHEAR ? 11 : 0] * wy;
+            acc[NW - 1] += c[SHEAR ? 11 : 0] * wx; acc[NW - 1] += c[SHEAR ? 12 : 0] * wy;
+          }
+        });
       });
     });
   });

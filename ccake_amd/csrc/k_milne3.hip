@@ -338,9 +338,11 @@ __device__ __forceinline__ Target3 target3(int n)
 // the list's reads from LDS (32 of its cycles a step, four SIMDs a CU).  A
 // smoothing pass of 100,007 particles (73 M pairs): 363 us with 64 targets a
 // tile and records in scalar registers, 212 us now.  MODE 2 the same way: the
-// count walked one candidate at a time took 1.7 ms.
+// count walked one candidate at a time took 1.7 ms.  The register budget keeps the
+// 5 waves per SIMD (4 in the other modes) that the walk has without its repeat for
+// sums that are not finite (for_tile_sums).
 template <int MODE, bool FACT, int W>
-__global__ __launch_bounds__(kWave * W) void k3_smooth_tile(const double* __restrict__ cand,
+__global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu((MODE == 0 && !FACT) ? 5 : 4))) void k3_smooth_tile(const double* __restrict__ cand,
                                                             const int32_t* __restrict__ skey,
                                                             const int32_t* __restrict__ cell_off,
                                                             const Grid* __restrict__ gridp, int n, double rc2,
@@ -362,53 +364,62 @@ __global__ __launch_bounds__(kWave * W) void k3_smooth_tile(const double* __rest
   const double m4h = -0.25 * hinv, mk2h = -0.5 * hinv * kSplineK;
   double* mine = list[t.slice];
 
-  double acc[5] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
-  int cnt = 0;
-  for_segments3(t.act, myrow, r, [&](const Seg3& seg, bool in) {
-    const double xs = in ? r[0] : kFarAway;
-    walk_tile3<W, NP>(g, cell_off, seg, rc2, rcs, t.slice,
-      [&](int j, double (&c)[NP]) {
-        #pragma unroll
-        for (int q = 0; q < NP; ++q) c[q] = cand[(size_t)j * kCandS + q];
-      },
-      [&](int e, const double (&c)[NP], int) {
-        #pragma unroll
-        for (int q = 0; q < NP; ++q) mine[e * NP + q] = c[q];
-      },
-      [&](int from, int to) {
-        #pragma unroll
-        for (int q = 0; q < NP; ++q) mine[to * NP + q] = mine[from * NP + q];
-      },
-      [&](int e) {
-        mine[e * NP] = -kFarAway;
-        #pragma unroll
-        for (int q = 1; q < NP; ++q) mine[e * NP + q] = 0.0;
-      },
-      [&](int e0, auto steps) {
-        #pragma unroll
-        for (int u = 0; u < decltype(steps)::value; ++u) {
-          const double* c = mine + (e0 + kGroups3 * u + t.group) * NP;
-          const double dx = xs - c[0], dy = r[1] - c[1], dz = r[2] - c[2];
-          const double r2 = dist2_3(dx, dy, dz);
-          const bool nb = r2 <= rc2;
-          cnt += nb ? 1 : 0;
-          if (MODE == 2) continue;
-          double w;
-          if (FACT) {
-            double qp, iqp, qe, iqe;
-            q_and_inverse(dist2_perp(dx, dy), hinv * hinv, qp, iqp);
-            q_and_inverse(dz * dz, heinv * heinv, qe, iqe);
-            w = nb ? spline_w(qp) * spline_w(qe) : 0.0;
+  double acc[5];
+  int cnt;
+  for_tile_sums<5>(acc, [&](auto in_range) {
+    cnt = 0;
+    for_segments3(t.act, myrow, r, [&](const Seg3& seg, bool in) {
+      const double xs = in ? r[0] : kFarAway;
+      walk_tile3<W, NP>(g, cell_off, seg, rc2, rcs, t.slice,
+        [&](int j, double (&c)[NP]) {
+          #pragma unroll
+          for (int q = 0; q < NP; ++q) c[q] = cand[(size_t)j * kCandS + q];
+        },
+        [&](int e, const double (&c)[NP], int) {
+          #pragma unroll
+          for (int q = 0; q < NP; ++q) mine[e * NP + q] = c[q];
+        },
+        [&](int from, int to) {
+          #pragma unroll
+          for (int q = 0; q < NP; ++q) mine[to * NP + q] = mine[from * NP + q];
+        },
+        [&](int e) {
+          mine[e * NP] = -kFarAway;
+          #pragma unroll
+          for (int q = 1; q < NP; ++q) mine[e * NP + q] = 0.0;
+        },
+        [&](int e0, auto steps) {
+          auto one = [&](int u) {
+            const double* c = mine + (e0 + kGroups3 * u + t.group) * NP;
+            const double dx = xs - c[0], dy = r[1] - c[1], dz = r[2] - c[2];
+            const double r2 = dist2_3(dx, dy, dz);
+            const bool nb = r2 <= rc2;
+            cnt += nb ? 1 : 0;
+            if (MODE == 2 || (decltype(in_range)::value && !nb)) return;
+            double w;
+            if (FACT) {
+              double qp, iqp, qe, iqe;
+              q_and_inverse(dist2_perp(dx, dy), hinv * hinv, qp, iqp);
+              q_and_inverse(dz * dz, heinv * heinv, qe, iqe);
+              w = nb ? spline_w(qp) * spline_w(qe) : 0.0;
+            } else {
+              w = spline_w8(r2, m4h, mk2h);
+            }
+            acc[0] += c[3] * w;
+            if (MODE == 0) {
+              #pragma unroll
+              for (int q = 1; q < 5; ++q) acc[q] += c[MODE == 0 ? 3 + q : 0] * w;
+            }
+          };
+          if (decltype(in_range)::value) {
+            #pragma unroll 1
+            for (int u = 0; u < decltype(steps)::value; ++u) one(u);
           } else {
-            w = spline_w8(r2, m4h, mk2h);
-          }
-          acc[0] += c[3] * w;
-          if (MODE == 0) {
             #pragma unroll
-            for (int q = 1; q < 5; ++q) acc[q] += c[MODE == 0 ? 3 + q : 0] * w;
+            for (int u = 0; u < decltype(steps)::value; ++u) one(u);
           }
-        }
-      });
+        });
+    });
   });
   // the four groups of the W waves, in order
   #pragma unroll
@@ -506,8 +517,44 @@ __device__ __forceinline__ void outer3(const double (&w)[3], double f, Sums3 (&a
 #endif
 }
 
+// The same on the targets that have the candidate in range (`nb`, of this lane's
+// target and candidate), and for_tile_sums for these sums.
+__device__ __forceinline__ void outer3_in_range(const double (&w)[3], double f, bool nb, Sums3 (&acc)[3])
+{
+  const int lane = threadIdx.x & (kWave - 1);
+  #pragma unroll 1
+  for (int k = 0; k < kGroups3; ++k) {
+    const double fk = __shfl(f, lane % kTile3 + kTile3 * k);
+    #pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int from = lane / kTile3 + 4 * r + kTile3 * k;
+      const int has = __shfl((int)nb, from);
+      #pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double wd = __shfl(w[d], from);
+        if (has) acc[d][r] += wd * fk;
+      }
+    }
+  }
+}
+template <class Walk>
+__device__ __forceinline__ void for_tile_sums(Sums3 (&acc)[3], Walk&& walk)
+{
+  const Sums3 none = { 0.0, 0.0, 0.0, 0.0 };
+  acc[0] = acc[1] = acc[2] = none;
+  walk(std::false_type());
+  double z = 0.0;
+  #pragma unroll
+  for (int q = 0; q < 12; ++q) z = fma(acc[q / 4][q % 4], 0.0, z);
+  if (__ballot(z != 0.0) == 0ull) return;
+  acc[0] = acc[1] = acc[2] = none;
+  walk(std::true_type());
+}
+
+// The register budget: 4 waves per SIMD, as without the repeat (which would
+// take 160 registers and leave 3).
 template <bool SHEAR, bool FACT, int W>
-__global__ __launch_bounds__(kWave * W) void k3_grad_tile(const double* __restrict__ cand,
+__global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4))) void k3_grad_tile(const double* __restrict__ cand,
                                                           const int32_t* __restrict__ skey,
                                                           const int32_t* __restrict__ cell_off,
                                                           const Grid* __restrict__ gridp, int n, double rc2,
@@ -530,55 +577,64 @@ __global__ __launch_bounds__(kWave * W) void k3_grad_tile(const double* __restri
   long long* off = reinterpret_cast<long long*>(buf[t.slice] + kList3 * NP);   // a record's first field
   const double* fields = cand + 4 + t.i;
 
-  Sums3 acc[3] = { { 0.0, 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0, 0.0 }, { 0.0, 0.0, 0.0, 0.0 } };
-  for_segments3(t.act, myrow, r, [&](const Seg3& seg, bool in) {
-    const double xs = in ? r[0] : kFarAway;
-    walk_tile3<W, NP>(g, cell_off, seg, rc2, rcs, t.slice,
-      [&](int j, double (&c)[NP]) {
-        #pragma unroll
-        for (int q = 0; q < NP; ++q) c[q] = cand[(size_t)j * kCandG3 + q];
-      },
-      [&](int e, const double (&c)[NP], int j) {
-        #pragma unroll
-        for (int q = 0; q < NP; ++q) pos[e * NP + q] = c[q];
-        off[e] = (long long)j * kCandG3;
-      },
-      [&](int from, int to) {
-        #pragma unroll
-        for (int q = 0; q < NP; ++q) pos[to * NP + q] = pos[from * NP + q];
-        off[to] = off[from];
-      },
-      [&](int e) {
-        pos[e * NP] = -kFarAway;
-        #pragma unroll
-        for (int q = 1; q < NP; ++q) pos[e * NP + q] = 0.0;
-        off[e] = off[0];
-      },
-      [&](int e0, auto steps) {
-        constexpr int U = decltype(steps)::value;
-        double f[U];
-        #pragma unroll
-        for (int u = 0; u < U; ++u) f[u] = fields[off[e0 + kGroups3 * u + t.group]];
-        #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const double* c = pos + (e0 + kGroups3 * u + t.group) * NP;
-          const double dx = xs - c[0], dy = r[1] - c[1], dz = r[2] - c[2];
-          double w[3];
-          if (FACT) {
-            double qp, iqp, qe, iqe;
-            q_and_inverse(dist2_perp(dx, dy), hinv * hinv, qp, iqp);
-            q_and_inverse(dz * dz, heinv * heinv, qe, iqe);
-            const double m = dist2_3(dx, dy, dz) <= rc2 ? c[3] : 0.0;
-            const double gp = m * spline_g(qp, iqp) * spline_w(qe);
-            w[0] = gp * dx; w[1] = gp * dy;
-            w[2] = m * kfac * spline_w(qp) * spline_g(qe, iqe) * dz;
-          } else {
-            const double gm = c[3] * spline_g2(fma(dx, dx, fma(dy, dy, dz * dz)), m4h, m2h);
-            w[0] = gm * dx; w[1] = gm * dy; w[2] = gm * dz;
+  Sums3 acc[3];
+  for_tile_sums(acc, [&](auto in_range) {
+    for_segments3(t.act, myrow, r, [&](const Seg3& seg, bool in) {
+      const double xs = in ? r[0] : kFarAway;
+      walk_tile3<W, NP>(g, cell_off, seg, rc2, rcs, t.slice,
+        [&](int j, double (&c)[NP]) {
+          #pragma unroll
+          for (int q = 0; q < NP; ++q) c[q] = cand[(size_t)j * kCandG3 + q];
+        },
+        [&](int e, const double (&c)[NP], int j) {
+          #pragma unroll
+          for (int q = 0; q < NP; ++q) pos[e * NP + q] = c[q];
+          off[e] = (long long)j * kCandG3;
+        },
+        [&](int from, int to) {
+          #pragma unroll
+          for (int q = 0; q < NP; ++q) pos[to * NP + q] = pos[from * NP + q];
+          off[to] = off[from];
+        },
+        [&](int e) {
+          pos[e * NP] = -kFarAway;
+          #pragma unroll
+          for (int q = 1; q < NP; ++q) pos[e * NP + q] = 0.0;
+          off[e] = off[0];
+        },
+        [&](int e0, auto steps) {
+          constexpr int U = decltype(steps)::value;
+          auto one = [&](int u, double f) {
+            const double* c = pos + (e0 + kGroups3 * u + t.group) * NP;
+            const double dx = xs - c[0], dy = r[1] - c[1], dz = r[2] - c[2];
+            double w[3];
+            if (FACT) {
+              double qp, iqp, qe, iqe;
+              q_and_inverse(dist2_perp(dx, dy), hinv * hinv, qp, iqp);
+              q_and_inverse(dz * dz, heinv * heinv, qe, iqe);
+              const double m = dist2_3(dx, dy, dz) <= rc2 ? c[3] : 0.0;
+              const double gp = m * spline_g(qp, iqp) * spline_w(qe);
+              w[0] = gp * dx; w[1] = gp * dy;
+              w[2] = m * kfac * spline_w(qp) * spline_g(qe, iqe) * dz;
+            } else {
+              const double gm = c[3] * spline_g2(fma(dx, dx, fma(dy, dy, dz * dz)), m4h, m2h);
+              w[0] = gm * dx; w[1] = gm * dy; w[2] = gm * dz;
+            }
+            if (decltype(in_range)::value) outer3_in_range(w, f, dist2_3(dx, dy, dz) <= rc2, acc);
+            else outer3(w, f, acc);
+          };
+          if (decltype(in_range)::value) {
+            #pragma unroll 1
+            for (int u = 0; u < U; ++u) one(u, fields[off[e0 + kGroups3 * u + t.group]]);
+            return;
           }
-          outer3(w, f[u], acc);
-        }
-      });
+          double f[U];
+          #pragma unroll
+          for (int u = 0; u < U; ++u) f[u] = fields[off[e0 + kGroups3 * u + t.group]];
+          #pragma unroll
+          for (int u = 0; u < U; ++u) one(u, f[u]);
+        });
+    });
   });
   #pragma unroll
   for (int d = 0; d < 3; ++d)

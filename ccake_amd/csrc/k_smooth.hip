@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kWave * W) void k_count_tile(const double* __restri
     const Grid& g = gridp[event_index(gridp, g0, seg.row)];
     const double xs = in ? xi : kFarAway;
     for_spans_slice<kCandS, false>(g, cell_off, cand, seg, rc2, rcs, slice, W, [&](RunCursor& cur) {
-      walk_records<2, kCandS, 1>(cand, xs, yi, cur, [&](const double*, double, double, double r2) {
+      walk_records<2, kCandS, false>(cand, xs, yi, rc2, cur, [&](const double*, double, double, double r2) {
         cnt += r2 <= rc2 ? 1 : 0;
       });
     });
@@ -205,37 +205,39 @@ __device__ __forceinline__ void smooth_walk(const double* __restrict__ cand, con
   const double xi = me[0], yi = me[1];
   const int myrow = act ? skey[kk] / g0.stride : INT_MAX;
 
-  double sl = 0.0, ss = 0.0, sB = 0.0, sS = 0.0, sQ = 0.0;
-  int cnt = 0;   // r2 <= rc2, the self pair included
-
-  for_segments(gridp, g0, FORM == kSmall ? rcs : 0.0, act, myrow, xi, yi, [&](const Seg& seg, bool in) {
-    const Grid& g = gridp[event_index(gridp, g0, seg.row)];
-    const double xs = in ? xi : kFarAway;      // lanes of other cell rows sit this segment's walk out
-    for_spans_slice<kCandS, FORM == kKeep>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
-      // whole records or half records: one scalar load each
-      constexpr int NR = (MODE == 0) ? 8 : 4;
-      walk_records<NR, kCandS, 1>(cand, xs, yi, cur,
-                               [&](const double* c, double dx, double dy, double r2) {
-        cnt += r2 <= rc2 ? 1 : 0;
-        double w;
-        if (FORM == kKeep) {
-          double q, iq;
-          q_and_inverse(r2, hinv2, q, iq);
-          w = spline_w(q);
-        } else {
-          w = spline_w8<FORM>(r2, m4h, mk2h);
-        }
-        sl += c[2] * w;
-        if (MODE == 0 || MODE == 3) ss += c[MODE == 1 ? 0 : 3] * w;
-        if (MODE == 0) {
-          sB += c[MODE == 0 ? 4 : 0] * w;
-          sS += c[MODE == 0 ? 5 : 0] * w; sQ += c[MODE == 0 ? 6 : 0] * w;
-        }
+  double sum[5];                   // sigma_lab, s, B, S, Q
+  int cnt;                         // r2 <= rc2, the self pair included
+  for_tile_sums<5>(sum, [&](auto in_range) {
+    cnt = 0;
+    for_segments(gridp, g0, FORM == kSmall ? rcs : 0.0, act, myrow, xi, yi, [&](const Seg& seg, bool in) {
+      const Grid& g = gridp[event_index(gridp, g0, seg.row)];
+      const double xs = in ? xi : kFarAway;      // lanes of other cell rows sit this segment's walk out
+      for_spans_slice<kCandS, FORM == kKeep>(g, cell_off, cand, seg, rc2, rcs, slice, nslices, [&](RunCursor& cur) {
+        // whole records or half records: one scalar load each
+        constexpr int NR = (MODE == 0) ? 8 : 4;
+        walk_records<NR, kCandS, decltype(in_range)::value>(cand, xs, yi, rc2, cur,
+                                 [&](const double* c, double dx, double dy, double r2) {
+          cnt += r2 <= rc2 ? 1 : 0;
+          double w;
+          if (FORM == kKeep) {
+            double q, iq;
+            q_and_inverse(r2, hinv2, q, iq);
+            w = spline_w(q);
+          } else {
+            w = spline_w8<FORM>(r2, m4h, mk2h);
+          }
+          sum[0] += c[2] * w;
+          if (MODE == 0 || MODE == 3) sum[1] += c[MODE == 1 ? 0 : 3] * w;
+          if (MODE == 0) {
+            sum[2] += c[MODE == 0 ? 4 : 0] * w;
+            sum[3] += c[MODE == 0 ? 5 : 0] * w; sum[4] += c[MODE == 0 ? 6 : 0] * w;
+          }
+        });
       });
     });
   });
   const double f = FORM == kKeep ? 1.0 : kSplineW;
-  const double acc[6] = { f * sl, (double)cnt, f * ss, f * sB, f * sS, f * sQ };
+  const double acc[6] = { f * sum[0], (double)cnt, f * sum[1], f * sum[2], f * sum[3], f * sum[4] };
   fin(acc);
 }
 

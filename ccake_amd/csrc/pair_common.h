@@ -8,6 +8,7 @@
 #pragma once
 #include "ccake_internal.h"
 #include <climits>
+#include <type_traits>
 
 namespace ccake {
 
@@ -254,7 +255,7 @@ struct RunCursor {
 // KEEP: contiguous all the same (keep_order).  body(cursor) once per 64 cell
 // rows that hold some of the slice.  Called with every lane of the wave
 // active; body runs on every lane (wave-uniform control flow): a lane outside
-// the segment stands at kFarAway, which every candidate's weight is 0 for.
+// the segment stands at kFarAway, where every candidate's weight is 0.
 template <int STRIDE, bool KEEP, class Body>
 __device__ __forceinline__ void for_spans_slice(const Grid& g, const int32_t* __restrict__ cell_off,
                                                 const double* __restrict__ cand, const Seg& s, double rc2, double rcs,
@@ -372,77 +373,82 @@ __device__ __forceinline__ void pin_scalar(const double (&r)[NR])
 #endif
 }
 
-// One step of walk_records: the U records of `cur` are evaluated (the first
-// alone when there is no second) while those at sorted indices n[] are
-// requested.  A wait on scalar loads covers every one in flight (they can
-// return out of order), so the wait for `cur` is taken by its offsets, before
-// the request (pin_vector), and the wait for `nxt` falls after the whole of
-// this step's arithmetic (pin_scalar: the compiler would otherwise move its
-// loads to their use in the next step).
-template <int NR, int STRIDE, int U, class Body>
-__device__ __forceinline__ void walk_step(const double (&cur)[U][NR], double (&nxt)[U][NR],
-                                          const double* __restrict__ cand, const int (&n)[U], bool whole, double xi,
-                                          double yi, Body&& body)
+// One step of walk_records: the record `cur` is evaluated while the one at
+// sorted index n is requested.  A wait on scalar loads covers every one in
+// flight (they can return out of order), so the wait for `cur` is taken by its
+// offsets, before the request (pin_vector), and the wait for `nxt` falls after
+// the whole of this step's arithmetic (pin_scalar: the compiler would otherwise
+// move its loads to their use in the next step).
+template <int NR, int STRIDE, class Body>
+__device__ __forceinline__ void walk_step(const double (&cur)[NR], double (&nxt)[NR], const double* __restrict__ cand,
+                                          int n, double xi, double yi, Body&& body)
 {
-  double dx[U], dy[U];
-  #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    dx[u] = xi - cur[u][0];
-    dy[u] = yi - cur[u][1];
-    pin_vector(dx[u], dy[u]);
-  }
+  double dx = xi - cur[0], dy = yi - cur[1];
+  pin_vector(dx, dy);
   __builtin_amdgcn_sched_barrier(0);
   #pragma unroll
-  for (int u = 0; u < U; ++u)
-    #pragma unroll
-    for (int q = 0; q < NR; ++q) nxt[u][q] = cand[(size_t)n[u] * STRIDE + q];
+  for (int q = 0; q < NR; ++q) nxt[q] = cand[(size_t)n * STRIDE + q];
   __builtin_amdgcn_sched_barrier(0);
-  #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (u == 0 || whole) body(cur[u], dx[u], dy[u], dist2_nocontract(dx[u], dy[u]));
-  #pragma unroll
-  for (int u = 0; u < U; ++u) pin_scalar<NR>(nxt[u]);
+  body(cur, dx, dy, dist2_nocontract(dx, dy));
+  pin_scalar<NR>(nxt);
 }
 
-// Walk the candidates of a cursor, their records in scalar registers, U at a
-// time (1 or 2) and the next U requested ahead into the other of two register
-// sets: with one set and a copy, the loads of a record cannot be issued
-// before the last use of the one it replaces, and every candidate waits for
-// its own loads.  body(c, dx, dy, r2) adds one candidate's terms.
-template <int NR, int STRIDE, int U, class Body>
-__device__ __forceinline__ void walk_records(const double* __restrict__ cand, double xi, double yi, RunCursor& cur,
-                                             Body&& body)
+// Walk the candidates of a cursor, their records in scalar registers, the next
+// one requested ahead into the other of two register sets: with one set and a
+// copy, the loads of a record cannot be issued before the last use of the one
+// it replaces, and every candidate waits for its own loads.  body(c, dx, dy,
+// r2) adds one candidate's terms.  IN_RANGE: only on the lanes that have it in
+// range, one record after the other (for_tile_sums).
+template <int NR, int STRIDE, bool IN_RANGE, class Body>
+__device__ __forceinline__ void walk_records(const double* __restrict__ cand, double xi, double yi, double rc2,
+                                             RunCursor& cur, Body&& body)
 {
-  static_assert(U == 1 || U == 2, "one or two records per step");
-  double a[U][NR], b[U][NR];
-  int n[U];                       // the next records' indices; a missing one repeats the one before (in bounds, unused)
-  int count;                      // how many of them there are
-  auto take = [&]() {
-    const int j = cur.next();
-    count = j < 0 ? 0 : 1;
-    if (j >= 0) n[0] = j;
-    if (U == 2) {
-      const int k = j < 0 ? -1 : cur.next();
-      count += k < 0 ? 0 : 1;
-      n[U - 1] = k < 0 ? n[0] : k;
+  if (IN_RANGE) {
+    for (int j = cur.next(); j >= 0; j = cur.next()) {
+      const double* c = cand + (size_t)j * STRIDE;
+      const double dx = xi - c[0], dy = yi - c[1], r2 = dist2_nocontract(dx, dy);
+      if (r2 <= rc2) body(c, dx, dy, r2);
     }
-  };
-  take();
-  if (count == 0) return;
-  #pragma unroll
-  for (int u = 0; u < U; ++u)
-    #pragma unroll
-    for (int q = 0; q < NR; ++q) a[u][q] = cand[(size_t)n[u] * STRIDE + q];
-  for (;;) {
-    bool whole = count == U;
-    take();
-    walk_step<NR, STRIDE, U>(a, b, cand, n, whole, xi, yi, body);
-    if (count == 0) break;
-    whole = count == U;
-    take();
-    walk_step<NR, STRIDE, U>(b, a, cand, n, whole, xi, yi, body);
-    if (count == 0) break;
+    return;
   }
+  double a[NR], b[NR];
+  int n = cur.next();             // the next record's index; past the last the one before stays (in bounds, unused)
+  if (n < 0) return;
+  #pragma unroll
+  for (int q = 0; q < NR; ++q) a[q] = cand[(size_t)n * STRIDE + q];
+  for (;;) {
+    int j = cur.next();
+    if (j >= 0) n = j;
+    walk_step<NR, STRIDE>(a, b, cand, n, xi, yi, body);
+    if (j < 0) break;
+    j = cur.next();
+    if (j >= 0) n = j;
+    walk_step<NR, STRIDE>(b, a, cand, n, xi, yi, body);
+    if (j < 0) break;
+  }
+}
+
+// The sums acc[NACC] of a tile's walk.  walk(in_range) adds every candidate's
+// terms to them: on every lane at first, the weight being 0 where the candidate
+// is out of range.  0 times NaN or infinity is not 0, though, and a tile can
+// hold targets that such a candidate has nothing to do with (out of its range,
+// another event's); so where a sum is not finite, the walk is done again with
+// each candidate's terms added by the lanes that have it in range alone.
+// (Masking every candidate of every walk: 188,250 particles, smoothing 610 ->
+// 649 us, gradients 965 -> 1,051; 7,650: 30 -> 37 and 50 -> 70.)
+template <int NACC, class Walk>
+__device__ __forceinline__ void for_tile_sums(double (&acc)[NACC], Walk&& walk)
+{
+  #pragma unroll
+  for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
+  walk(std::false_type());
+  double z = 0.0;                  // stays 0 while every sum is finite
+  #pragma unroll
+  for (int q = 0; q < NACC; ++q) z = fma(acc[q], 0.0, z);
+  if (__ballot(z != 0.0) == 0ull) return;
+  #pragma unroll
+  for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
+  walk(std::true_type());
 }
 
 // q = r/h and 1/q from r^2: the hardware reciprocal square root
@@ -489,8 +495,8 @@ __device__ __forceinline__ double spline_g(double q, double iq)
 // spline_g(q, 1/q) = 2 h (t^2 - u^2) (2 / r) and
 // spline_w(q) = 8 (t^3 - (k u)^3), k = 2^(-1/3): the clamps make the cut at
 // 2h and the switch at h.  The walks apply the factors 2 h and 8 once per
-// particle.  A lane whose position is kFarAway gets exactly 0 from every
-// candidate (r^2 = 1e200 stays finite).
+// particle.  A lane whose position is kFarAway weighs every candidate exactly 0
+// (r^2 = 1e200 stays finite).
 constexpr double kFarAway = 1e100;
 constexpr double kSplineW = 8.0;                     // spline_w / spline_w8
 __device__ __forceinline__ double clamp01(double v) { return fmin(fmax(v, 0.0), 1.0); }

@@ -88,6 +88,23 @@ def test_batch_on_host_emulation(emu_lib):
     assert "OK" in r.stdout
 
 
+@pytest.mark.parametrize("args", [("small",), ("small", "4"), ("small", "2"), ("recorded",), ("mixed",), ("diffusion",),
+                                  ("milne",), ("milne_fact", "1")])
+def test_a_non_finite_value_stays_within_its_range(emu_lib, args):
+    """Two events (1,070 and 864 particles) in a batch, or a 3+1D event (864), one
+    particle with NaN or infinity in its bulk pressure, shear stress, entropy,
+    diffusion current or velocity (0 times either is NaN): a particle out of its
+    range, and the batch's second event, whose first rows share a tile with the
+    first event's last, keep their fields bit for bit, in each form of the pair
+    walks."""
+    env = dict(os.environ)
+    r = subprocess.run(["bash", os.path.join(EMU, "emu.sh"), os.path.join(EMU, "run_nonfinite.py"), *args],
+                       capture_output=True, text=True, timeout=600, env=env)
+    print(r.stdout[-4000:], r.stderr[-8000:])
+    assert r.returncode == 0 and "AddressSanitizer" not in r.stderr
+    assert r.stdout.rstrip().endswith("OK")
+
+
 def test_private_columns_disjoint():
     """Every multi-column private member owns its columns (the overlap that
     wrote past the field buffer is gone): parse the enumeration and check
