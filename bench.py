@@ -362,7 +362,7 @@ def large_batch(dev, eos, cfg, k, sample=32, seed=0xC3):
     n = [len(d["x"]) for d in ics]
     ntot = int(sum(n))
     print(f"bench: {ntot} particles; autotune", file=sys.stderr, flush=True)
-    tune = batching.autotune(dev, eos, dict(cfg, pair_precision=1), ics, cells_per_rc=(3, 4), slices=(1, 2, 4))
+    tune = batching.autotune(dev, eos, dict(cfg, pair_precision=1), ics, cells_per_rc=(3, 4), slices=(1, 2, 4, 8))
     print(f"bench: autotune {json.dumps(tune)}; plain path on {sample} events", file=sys.stderr, flush=True)
     alone = batching.run_alone(dev, eos, cfg, ics[:sample])
     plain = batching.latency_summary(alone, int(sum(n[:sample])))

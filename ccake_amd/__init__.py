@@ -421,7 +421,8 @@ class Event:
 
     def nslices(self, set_to=0):
         """Slices per tile of the pair kernels; set_to > 0 changes it (up to
-        the count the event was created with)."""
+        the count the event was created with, which runs the kernels' own
+        split)."""
         v = C.c_int()
         _ok(lib().ccake_event_pair_slices(self.h, int(set_to), C.byref(v)), "pair_slices")
         return v.value

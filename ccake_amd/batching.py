@@ -54,8 +54,9 @@ def make_batch(dev, eos, cfg, ics):
 def autotune(dev, eos, cfg, ics, cells_per_rc=(2, 3, 4), slices=(4, 8, 12, 16), steps=2):
     """Cell size and work per wave for a batch: for each cells-per-radius
     candidate a batch of the events is initialized and stepped twice, then
-    every slice count (pair-kernel waves per tile) is timed over `steps`
-    steps; the fastest pair is returned with the table of timings
+    every slice count (pair-kernel waves per tile) up to the one the batch was
+    created with, or that one where it is below them all, is timed over
+    `steps` steps; the fastest pair is returned with the table of timings
     (ms per step).  The tuning batches are discarded."""
     table = {}
     best = None
@@ -64,9 +65,7 @@ def autotune(dev, eos, cfg, ics, cells_per_rc=(2, 3, 4), slices=(4, 8, 12, 16), 
         b.initialize()
         b.run_steps(cfg["dt"], 2)
         cap = b.nslices()
-        for s in slices:
-            if s > cap:
-                continue
+        for s in [q for q in slices if q <= cap] or [cap]:
             b.nslices(s)
             b.run_steps(cfg["dt"], 1)
             dev.sync()

@@ -739,12 +739,11 @@ static int event_create(ccake_dev* dev, const ccake_params* p, ccake_eos* eos, i
   rc |= dalloc(ev, &ev->scan_tmp, (size_t)nscan_blocks);
   rc |= dalloc(ev, &ev->cell_off, (size_t)ev->cap_cells + 1);
   rc |= dalloc(ev, &ev->pair_count, 2);
-  const int cap = choose_slices((n + kTile - 1) / kTile, dev->simds);
-  ev->nslices = p->dim == 3 ? kTileWaves3 : kTileWaves;
-  bool sized = false;
+  ev->nslices = choose_slices((n + kTile - 1) / kTile, dev->simds);
+  ev->own_slices = true;
   if (const char* ov = std::getenv("CCAKE_PAIR_SLICES")) {     // tuning override, 1..16
     const int v = std::atoi(ov);
-    if (v >= 1 && v <= kMaxSlices) { ev->nslices = v; sized = true; }
+    if (v >= 1 && v <= kMaxSlices) { ev->nslices = v; ev->own_slices = false; }
   }
   if (const char* ov = std::getenv("CCAKE_LDS_SLICES"))        // tuning override: 0 sums slices through HBM
     ev->lds_reduce = std::atoi(ov) != 0;
@@ -752,12 +751,9 @@ static int event_create(ccake_dev* dev, const ccake_params* p, ccake_eos* eos, i
     const double v = std::atof(ov);
     if (v >= 0.0 && v <= 1.0) ev->skin_frac = v;
   }
-  ev->nslices_cap = std::max(ev->nslices, cap);
-  // partial sums: 17 per slice in 2+1D, the smoothing sums in 3+1D.  Tile
-  // workgroups store one slice's, so their 8 waves need no more room than the
-  // slices an event of this size would take.
-  ev->part_slices = ev->lds_reduce && !sized ? cap : ev->nslices_cap;
-  rc |= dalloc(ev, &ev->part, (p->dim == 3 ? (size_t)6 : (size_t)ev->part_slices * kMaxAcc) * np);
+  ev->nslices_cap = ev->nslices;
+  // partial sums: 17 per slice in 2+1D, the smoothing sums in 3+1D (whose tiles store one slice's)
+  rc |= dalloc(ev, &ev->part, (p->dim == 3 ? (size_t)6 : (size_t)ev->nslices_cap * kMaxAcc) * np);
   rc |= dalloc(ev, &ev->hard, np);
   {
     // the EoS stage in two kernels (table chains): CCAKE_EOS_SPLIT=0 keeps one
@@ -1264,8 +1260,7 @@ int ccake_event_pair_slices(ccake_event* ev, int set, int* nslices)
 {
   if (!ev) return CCAKE_ERR_INVALID;
   if (set > 0) {
-    const bool stored = ev->p.dim == 2 && !(ev->lds_reduce && set >= 4);   // every slice's sums go to the buffer
-    if (set > ev->nslices_cap || (stored && set > ev->part_slices)) { set_error("slice count above the event's partial-sum capacity"); return CCAKE_ERR_INVALID; }
+    if (set > ev->nslices_cap) { set_error("slice count above the event's partial-sum capacity"); return CCAKE_ERR_INVALID; }
     ev->nslices = set;
   }
   if (nslices) *nslices = ev->nslices;

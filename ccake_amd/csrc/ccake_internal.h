@@ -180,8 +180,8 @@ struct ccake_event {
   int init_phase = 0;               // initialisation phases done (1, 2, 3)
   // pair-kernel partial sums: nslices x (up to 17) x npad, sorted order
   int nslices = 1;
-  int nslices_cap = 1;          // largest slice count the event accepts
-  int part_slices = 1;          // slices the partial-sum buffer holds
+  int nslices_cap = 1;          // the count the event was created with: the buffer holds that many
+  bool own_slices = true;       // that count is the library's choice (pair_waves)
   // EoS stage: particles whose inversion needs the full cascade (positions),
   // two alternating counters and which one the next stage appends to
   double* k4 = nullptr;         // RK4 accumulator (allocated at the first fourth-order step)
@@ -255,13 +255,32 @@ inline double search_radius(const ccake_event* ev)
 }
 inline int32_t* icol(ccake_event* ev, int f) { return ev->I + (size_t)f * ev->npad; }
 
+// Slices of a tile that are walked side by side.  A count that the caller set is
+// taken as it is.  The one the event was created with is what its buffer of
+// partial sums holds; a tile's waves that add their slices in LDS store one
+// slice's sums whatever their number, so they are as many as measured best.
+// 2+1D: more do not pay even where 8 leave SIMDs empty (2,601 particles, 41
+// tiles: smoothing and gradients 55 us a stage with 8, 58 with 16), and 16
+// cost where they do not (30,300 particles: 128 against 142 us).
+constexpr int kTileWaves = 8;
+// 3+1D, tiles of 16 targets: smoothing and gradients 662 us a stage with 1 wave,
+// 608 with 2, 602 with 4 at 100,007 particles; 172, 146 and 134 at 25,018.
+constexpr int kTileWaves3 = 4;
+inline int pair_waves(const ccake_event* ev)
+{
+  const bool chosen = !ev->own_slices || ev->nslices != ev->nslices_cap;
+  if (chosen || (ev->p.dim == 2 && !ev->lds_reduce)) return ev->nslices;
+  return ev->p.dim == 3 ? kTileWaves3 : kTileWaves;
+}
+
 // Waves per workgroup of the 2+1D pair kernels that add a tile's slices in
 // LDS (one wave per slice), or 0 for one single-wave workgroup per (tile,
 // slice) with the slices' sums through HBM.
 inline int lds_slices(const ccake_event* ev)
 {
   if (ev->p.dim != 2 || !ev->lds_reduce) return 0;
-  return ev->nslices >= 8 ? 8 : (ev->nslices >= 4 ? 4 : 0);
+  const int w = pair_waves(ev);
+  return w >= 8 ? 8 : (w >= 4 ? 4 : 0);
 }
 
 // ---- launchers (one per .hip unit) ----

@@ -15,6 +15,7 @@
 //    17 neighbour-side sums of w = m_b grad W_ab and the sum pass applies
 //    the owner terms (and v_a) once.
 #include "pair_common.h"
+#include <algorithm>
 
 namespace ccake {
 
@@ -240,7 +241,7 @@ int launch_diff_grad(ccake_event* ev)
   const double h = ev->p.hT;
   const double rc = 2.0 * h;
   const int ntiles = (n + kTile - 1) / kTile;
-  const int slices = ev->nslices < ev->part_slices ? ev->nslices : ev->part_slices;   // each slice's sums are stored
+  const int slices = std::min(pair_waves(ev), ev->nslices_cap);   // each slice's sums are stored
   hipLaunchKernelGGL(k_diff_slice, dim3(ntiles * slices), dim3(kWave), 0, ev->stream, ev->cand_d, ev->skey,
                      ev->cell_off, ev->grid, n, rc * rc, search_radius(ev), -0.25 / h, -0.5 / h, slices, ev->part,
                      ev->npad);

@@ -1186,7 +1186,11 @@ double smooth_norm2_event(const ccake_event* ev)
 }
 
 // Waves per tile: the event's slices, as far as there are variants.
-static int tile3_waves(const ccake_event* ev) { return ev->nslices >= 4 ? 4 : (ev->nslices >= 2 ? 2 : 1); }
+static int tile3_waves(const ccake_event* ev)
+{
+  const int w = pair_waves(ev);
+  return w >= 4 ? 4 : (w >= 2 ? 2 : 1);
+}
 
 int launch3_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
 {

@@ -305,8 +305,9 @@ __device__ __forceinline__ void for_spans_slice(const Grid& g, const int32_t* __
 
 // Number of slices per tile for `ntiles` tiles on `simds` SIMDs: the
 // smallest that gives near-whole rounds of single-wave work units and at
-// least about four waves per SIMD (to hide load latency), at most 16.  It sets
-// how many slices an event accepts (ccake_event_pair_slices).
+// least about four waves per SIMD (to hide load latency), at most 16.  An event
+// is created with that count (ccake_event_pair_slices), and its buffer of partial
+// sums sized for it.
 inline int choose_slices(int ntiles, int simds)
 {
   int best = 1;
@@ -320,14 +321,6 @@ inline int choose_slices(int ntiles, int simds)
   return best;
 }
 
-// Slices per tile of the 2+1D kernels, which run a tile's slices as the waves
-// of one workgroup.  More do not pay even where 8 leave SIMDs empty (2,601
-// particles, 41 tiles: smoothing and gradients 55 us a stage with 8, 58 with
-// 16), and 16 cost where they do not (30,300 particles: 128 against 142 us).
-constexpr int kTileWaves = 8;
-// 3+1D, tiles of 16 targets: smoothing and gradients 662 us a stage with 1 wave,
-// 608 with 2, 602 with 4 at 100,007 particles; 172, 146 and 134 at 25,018.
-constexpr int kTileWaves3 = 4;
 // The gradient walk's waves are longer: 4 once they fill the SIMDs (188,250
 // particles, 2,942 tiles: 965 us with 4, 974 with 8; 182,355 in six events:
 // 349 against 369; 40,401 particles, 632 tiles: 96 us with 4, 89 with 8).

@@ -428,7 +428,10 @@ CCAKE_API int  ccake_pair_total(ccake_event* ev, int reset, int64_t* n_pairs);
 /* Slices per tile of the pair kernels (the work split of the smoothing and
  * gradient passes).  set > 0 chooses a new count, at most the count the
  * event was created with (its partial-sum buffer is sized for that); the
- * current count is returned in *nslices.  Results do not depend on it beyond
+ * current count is returned in *nslices.  With the count it was created
+ * with an event runs the kernels' own split (8 waves per tile in 2+1D, 4 in
+ * 3+1D); of a smaller one 2+1D uses 8, 4 or fewer, 3+1D 4, 2 or 1.
+ * Results do not depend on it beyond
  * summation order.  Tuning; no counterpart in the reference. */
 CCAKE_API int  ccake_event_pair_slices(ccake_event* ev, int set, int* nslices);
 

@@ -105,6 +105,17 @@ def test_a_non_finite_value_stays_within_its_range(emu_lib, args):
     assert r.stdout.rstrip().endswith("OK")
 
 
+def test_slice_counts(emu_lib):
+    """An event or batch takes every slice count up to the one it was created
+    with, which is the one it reports, and refuses those above."""
+    env = dict(os.environ)
+    r = subprocess.run(["bash", os.path.join(EMU, "emu.sh"), os.path.join(EMU, "run_slices.py")],
+                       capture_output=True, text=True, timeout=600, env=env)
+    print(r.stdout[-4000:], r.stderr[-8000:])
+    assert r.returncode == 0 and "AddressSanitizer" not in r.stderr
+    assert r.stdout.rstrip().endswith("OK")
+
+
 def test_private_columns_disjoint():
     """Every multi-column private member owns its columns (the overlap that
     wrote past the field buffer is gone): parse the enumeration and check

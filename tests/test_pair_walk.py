@@ -10,7 +10,7 @@ import pytest
 from scipy.spatial import cKDTree
 
 import ccake_amd  # noqa: F401
-from ccake_amd import config
+from ccake_amd import batching, config
 from parity_metrics import DERIVS, STATE
 from test_gpu_parity import Pair, compare, ints_equal
 from test_milne3 import DERIVS3, STATE3, Pair3, compare3
@@ -132,7 +132,8 @@ def test_single_precision_weights(dev, slices, shear):
 # are 4,096 tiles: whole rounds of the chip's SIMDs) runs its tiles of 8 waves in
 # no more device memory: the diffusion pass, which stores every slice's sums,
 # then takes one slice, and a slice count whose sums would not fit is refused.
-def test_partial_sums_fit(dev):
+# The autotuner takes what it is given as far as that goes.
+def test_partial_sums_fit(dev, monkeypatch):
     n = 262144
     m = 512
     x, y = (a.ravel() for a in np.meshgrid(np.arange(m) * 0.1, np.arange(m) * 0.1))
@@ -142,21 +143,28 @@ def test_partial_sums_fit(dev):
     e = 10.0 + np.cos(0.1 * x) + np.cos(0.1 * y)
     d = dict(x=x, y=y, e=e, ux=0.05 * np.sin(0.2 * x), uy=0.05 * np.sin(0.3 * y), rhoB=f * e, rhoS=0.5 * f * e, rhoQ=-f * e)
     eos = ccake_amd.Eos(dev, 0, 0.75)
-    ev = ccake_amd.Event(dev, eos, cfg, n)
-    ccake_amd.load_event(ev, d)
-    assert ev.nslices() == 8
-    ev.initialize()
-    ev.get_time_derivatives()
-    a = [ev.download(ccake_amd.FIELDS["CCAKE_F_" + f]) for f in ("GRADP0", "GRADV0", "DEXT_Q0")]
-    ev.nslices(4)
-    for s in (2, 3, 16):
-        with pytest.raises(RuntimeError):
-            ev.nslices(s)
-    ev.nslices(1)
-    ev.get_time_derivatives()
-    for u, v in zip(a, (ev.download(ccake_amd.FIELDS["CCAKE_F_" + f]) for f in ("GRADP0", "GRADV0", "DEXT_Q0"))):
+    a = []
+    for one in (False, True):
+        if one:                                  # one wave per tile
+            monkeypatch.setenv("CCAKE_PAIR_SLICES", "1")
+        ev = ccake_amd.Event(dev, eos, cfg, n)
+        ccake_amd.load_event(ev, d)
+        assert ev.nslices() == 1
+        for s in (2, 3, 4, 16):
+            with pytest.raises(RuntimeError):
+                ev.nslices(s)
+        ev.nslices(1)
+        ev.initialize()
+        ev.get_time_derivatives()
+        a.append([ev.download(ccake_amd.FIELDS["CCAKE_F_" + f]) for f in ("GRADP0", "GRADV0", "DEXT_Q0")])
+        ev.close()
+    monkeypatch.delenv("CCAKE_PAIR_SLICES")
+    for u, v in zip(*a):
         assert np.max(np.abs(u - v)) <= 1e-12 * np.max(np.abs(u)) > 0.0
-    ev.close()
+    assert any(np.any(u != v) for u, v in zip(*a))      # the tile's eight waves ran, then one
+    for slices in ((1, 2, 4), (4, 8)):
+        t = batching.autotune(dev, eos, dict(cfg, using_diffusion=0, pair_precision=1), [d], cells_per_rc=(4,), slices=slices, steps=1)
+        assert t["slices"] == 1
     eos.close()
 
 
