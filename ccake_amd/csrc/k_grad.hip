@@ -212,7 +212,7 @@ int launch_grad_pairs(ccake_event* ev)
     const std::integral_constant<int, 4> w4;
     if (single && W == 8) form(w8, std::integral_constant<int, kSingle>());
     else if (single) form(w4, std::integral_constant<int, kSingle>());
-    else if (W >= 2 * kKeepGradWaves && keep_order(ev, ntiles))
+    else if (W >= 2 * kKeepGradWaves && keep_order(ev))
       form(std::integral_constant<int, kKeepGradWaves>(), std::integral_constant<int, kKeep>());
     else if (W == 8 && small_event(ev, ntiles)) form(w8, std::integral_constant<int, kSmall>());
     else if (W == 8) form(w8, std::integral_constant<int, kExact>());

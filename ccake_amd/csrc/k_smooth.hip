@@ -392,7 +392,7 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
   const int m = (mode == 0 && ev->no_charges) ? 3 : mode;
   // the initial sigma stays in FP64 with pair_precision 1
   const bool single = mode == 0 && ev->p.pair_precision == 1;
-  const bool keep = !single && W >= kKeepSmoothWaves && keep_order(ev, ntiles);
+  const bool keep = !single && W >= kKeepSmoothWaves && keep_order(ev);
   const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT), m4h = (single ? -0.5 : -0.25) / ev->p.hT;
   const double mk2h = (single ? -1.0 : -0.5) * kSplineK / ev->p.hT;
   if (W) {

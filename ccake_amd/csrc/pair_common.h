@@ -326,22 +326,24 @@ inline int choose_slices(int ntiles, int simds)
 // 349 against 369; 40,401 particles, 632 tiles: 96 us with 4, 89 with 8).
 inline int grad_tile_waves(int waves, int ntiles, int simds) { return waves == 8 && ntiles >= simds ? 4 : waves; }
 
-// A small event whose freeze-out hypersurface is recorded keeps one order and
-// one form of its pair sums: the hypersurface's divE column is the
-// reciprocal of a difference, so another rounding of the sums moves its worst
-// entries by 1e-11 to 2e-9 after the 300 steps to freeze-out (10 events of
-// 5,000 to 7,650 particles), and runs of it are compared entry by entry.
-// While the waves do not fill the chip a pass is the latency of its setup and
-// loads, and the shorter arithmetic gains little: smoothing and gradients of
-// 7,650 particles take 31 and 51 us in this form, 30 and 40 in the other with
-// 8 waves per tile.
-inline bool keep_order(const ccake_event* ev, int ntiles)
-{
-  return ev->snaps && 8 * ntiles <= ev->dev->simds;
-}
-constexpr int kKeepSmoothWaves = 8, kKeepGradWaves = 4;
 // An event (or batch) of at most a wave per SIMD (for_segments).
 inline bool small_event(const ccake_event* ev, int ntiles) { return 8 * ntiles <= ev->dev->simds; }
+// A small event or batch in FP64 whose freeze-out hypersurface is recorded
+// (keep_order) has an order and a form of its pair sums of its own, kKeep, that
+// of the hypersurfaces recorded so far: their divE column is the reciprocal of a
+// difference, so another rounding of the sums moves its worst entries by 1e-11
+// to 2e-9 after the 300 steps to freeze-out (10 events of 5,000 to 7,650
+// particles), and they are compared entry by entry.  Events beyond that size
+// have the common form.  While the waves do not fill the chip a pass is the
+// latency of its setup and loads, and the shorter arithmetic gains little:
+// smoothing and gradients of 7,650 particles take 31 and 48 us in this form,
+// 30 and 40 in the other with 8 waves per tile.  The size is the one the event was
+// created with: a batch stays with its form while its events retire.
+inline bool keep_order(const ccake_event* ev)
+{
+  return ev->snaps && small_event(ev, (ev->n + kTile - 1) / kTile);
+}
+constexpr int kKeepSmoothWaves = 8, kKeepGradWaves = 4;
 
 // Per-slice partial sums: part[(slice * nacc + f) * npad + k] for sorted
 // position k (every tile lane, k < ntiles * 64 <= npad, has a slot).

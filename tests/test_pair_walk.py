@@ -168,6 +168,37 @@ def test_partial_sums_fit(dev, monkeypatch):
     eos.close()
 
 
+# A recorded batch above the kept order's 8,192 particles whose second event ends,
+# which leaves less than that: the first event goes on in the form it began with,
+# so as it does beside an event that has not ended.  (Its rows of 128 particles are
+# whole tiles, so that its tiles and their segments are the same either way.)
+def test_a_batch_keeps_its_form_as_events_end(dev):
+    def lines(nx, ny, gev):
+        x, y = (a.ravel() for a in np.meshgrid((np.arange(nx) - 0.5 * nx) * 0.05, np.arange(ny) * 0.15))
+        e = gev * (1.0 + 0.2 * np.cos(x) * np.cos(y)) / config.HBARC_GEVFM
+        z = np.zeros_like(x)
+        return dict(x=x, y=y, e=e, ux=0.1 * np.sin(x), uy=0.1 * np.sin(y), rhoB=0.02 * e, rhoS=z, rhoQ=z)
+
+    T = 150.0 / config.HBARC_MEVFM
+    eos = ccake_amd.Eos(dev, 0, T)
+    cfg = dict(config.lumpy_params(), particlization=1, e_freeze=eos.efreeze(T), cells_per_rc=4, x_subcells=8)
+    got = []
+    for gev in (0.2, 20.0):                          # the second event: cold, or as hot as the first
+        ics = [lines(128, 50, 20.0), lines(128, 20, gev)]
+        b = ccake_amd.Batch(dev, eos, cfg, [6400, 2560])
+        ccake_amd.load_event(b, ccake_amd.concat_ics(ics))
+        b.initialize()
+        for _ in range(12):
+            live = b.batch_continue_evolution(max_tau=30.0)
+            b.advance_timestep(cfg["dt"], 2)
+        got.append([bool(q) for q in live])
+        got.append(np.stack([b.download(ccake_amd.FIELDS["CCAKE_F_" + f])[:6400] for f in ("UX", "UY", "E", "GRADP0", "GRADV0")]))
+        b.close()
+    eos.close()
+    assert got[0] == [True, False] and got[2] == [True, True]
+    assert np.array_equal(got[1], got[3])
+
+
 # NaN or infinity in one particle stays within its range (0 times either is NaN):
 # the walks of the tiles that meet it are done again; 3+1D sums are then formed
 # outside the matrix cores, so in another order (a few hundred terms: 1e-13), and
