@@ -189,15 +189,14 @@ def bytes_per_particle_eos(nslices):
 
 
 KERNEL_OF_GROUP = {"SMOOTH": "k_smooth_slice", "GRAD": "k_grad_slice", "EOS": "k_eos"}
-# With 4 or more slices per tile the FP64 2+1D pair kernels run a tile's
-# slices as the waves of one workgroup and add them in LDS (k_smooth_tile,
-# k_grad_tile; CCAKE_LDS_SLICES=0 turns that off), and the sum passes read
-# one slice.
+# The 2+1D pair kernels run a tile's slices as the waves of one workgroup and
+# add them in LDS (k_smooth_tile, k_grad_tile; CCAKE_LDS_SLICES=0 turns that
+# off, as does a CCAKE_PAIR_SLICES below 4), and the sum passes read one slice.
 KERNEL_OF_GROUP_LDS = {"SMOOTH": "k_smooth_tile", "GRAD": "k_grad_tile", "EOS": "k_eos"}
 
 
 def lds_tiles(nslices, cfg):
-    return (nslices >= 4 and cfg.get("pair_precision", 0) == 0 and cfg.get("dim", 2) == 2
+    return ((nslices >= 4 or "CCAKE_PAIR_SLICES" not in os.environ) and cfg.get("dim", 2) == 2
             and os.environ.get("CCAKE_LDS_SLICES", "1") != "0")
 
 

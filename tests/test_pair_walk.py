@@ -170,18 +170,21 @@ def test_partial_sums_fit(dev, monkeypatch):
 
 # A recorded batch above the kept order's 8,192 particles whose second event ends,
 # which leaves less than that: the first event goes on in the form it began with,
-# so as it does beside an event that has not ended.  (Its rows of 128 particles are
-# whole tiles, so that its tiles and their segments are the same either way.)
-def test_a_batch_keeps_its_form_as_events_end(dev):
+# so as it does beside an event that has not ended.  (Its lines of 128 particles
+# are whole tiles, each in a cell row of its own, sorted anew in every stage, so
+# that its tiles and their segments are the same either way.)
+def test_a_batch_keeps_its_form_as_events_end(dev, monkeypatch):
     def lines(nx, ny, gev):
-        x, y = (a.ravel() for a in np.meshgrid((np.arange(nx) - 0.5 * nx) * 0.05, np.arange(ny) * 0.15))
+        x, y = (a.ravel() for a in np.meshgrid((np.arange(nx) - 0.5 * nx) * 0.05, np.arange(ny) * 0.45))
+        y[y > 0.0] += 0.075                          # the first line is the box's edge, the others mid-cell
         e = gev * (1.0 + 0.2 * np.cos(x) * np.cos(y)) / config.HBARC_GEVFM
         z = np.zeros_like(x)
         return dict(x=x, y=y, e=e, ux=0.1 * np.sin(x), uy=0.1 * np.sin(y), rhoB=0.02 * e, rhoS=z, rhoQ=z)
 
+    monkeypatch.setenv("CCAKE_SORT_SKIN", "0")
     T = 150.0 / config.HBARC_MEVFM
     eos = ccake_amd.Eos(dev, 0, T)
-    cfg = dict(config.lumpy_params(), particlization=1, e_freeze=eos.efreeze(T), cells_per_rc=4, x_subcells=8)
+    cfg = dict(config.lumpy_params(dt=0.002), particlization=1, e_freeze=eos.efreeze(T), cells_per_rc=4, x_subcells=8)
     got = []
     for gev in (0.2, 20.0):                          # the second event: cold, or as hot as the first
         ics = [lines(128, 50, 20.0), lines(128, 20, gev)]
@@ -196,6 +199,7 @@ def test_a_batch_keeps_its_form_as_events_end(dev):
         b.close()
     eos.close()
     assert got[0] == [True, False] and got[2] == [True, True]
+    print("differ by", np.max(np.abs(got[1] - got[3]), axis=1))
     assert np.array_equal(got[1], got[3])
 
 
