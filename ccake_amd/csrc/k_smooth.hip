@@ -393,8 +393,8 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
   // the initial sigma stays in FP64 with pair_precision 1
   const bool single = mode == 0 && ev->p.pair_precision == 1;
   const bool keep = !single && W >= kKeepSmoothWaves && keep_order(ev);
-  const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT), m4h = (single ? -0.5 : -0.25) / ev->p.hT;
-  const double mk2h = (single ? -1.0 : -0.5) * kSplineK / ev->p.hT;
+  const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT);
+  const double m4h = (single ? -0.5 / (1.0 + kSqrtMean) : -0.25) / ev->p.hT, mk2h = 2.0 * kSplineK * m4h;
   if (W) {
     // the tile's slices reduced in LDS: the sum pass sees one slice
     ev->smooth_sum_slices = 1;

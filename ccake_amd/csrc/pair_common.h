@@ -497,13 +497,20 @@ constexpr double kSplineW = 8.0;                     // spline_w / spline_w8
 __device__ __forceinline__ double clamp01(double v) { return fmin(fmax(v, 0.0), 1.0); }
 // FORM of a walk: kExact with the arithmetic above; kKeep with that of
 // q_and_inverse, spline_w and spline_g (keep_order); kSingle without the
-// Newton step (pair_precision 1): y and f as they are, so r and 1/r instead of
-// 2 r and 2 / r, with v_rsq_f64's relative error (5.2e-8 at most, 1.0e-8
-// rms over 4M arguments: less than one rounding to single precision),
+// Newton step (pair_precision 1): r and 1/r instead of 2 r and 2 / r, from y and
+// f as they are (v_rsq_f64: relative error 5.2e-8 at most, 1.0e-8 rms over 4M
+// arguments, less than one rounding to single precision) or, where 1/r is not
+// needed, r from v_sqrt_f64 (2.7e-8 and 8.4e-9), which takes 0 as it is;
 // everything else in FP64.  Single-precision arithmetic would not be faster: it
-// issues at the FP64 rate here.  188,250 particles: smoothing 615 -> 583 us,
-// gradients 968 -> 915 us (pair terms in FP32 with compensated sums: 557 and 986).  The constants m4h
-// and m2h (mk2h) are then twice as large, and the gradient's final factor.
+// issues at the FP64 rate here.  188,250 particles: smoothing 612 us in FP64, 547
+// (580 with r from v_rsq_f64), gradients 970 and 910 (pair terms in FP32 with
+// compensated sums: 548 and 990); 751,500: 8.0 and 7.1 ms (7.6; 7.2), 13.0 and
+// 12.1 (12.6).  The constants m4h and m2h (mk2h) are then twice as large, and the
+// gradient's final factor.  What does not average out over the pairs, the errors'
+// mean with the weight that a pair's r has in a density or a gradient, is taken
+// out by the constants: it is -3.3e-9 for v_sqrt_f64 (-3.1e-9 to -3.5e-9 for h
+// from 0.1 to 1) and 3.3e-9 for v_rsq_f64 (2.5e-9 to 4.0e-9), as measured.
+constexpr double kSqrtMean = -3.3e-9, kRsqMean = 3.3e-9;
 // kSmall: kExact with the rows of a tile as one segment where that reaches less
 // (for_segments), for events whose waves do not fill the SIMDs.
 enum Form { kExact, kKeep, kSingle, kSmall };
@@ -536,8 +543,9 @@ constexpr double kSplineK = 0.79370052598409973738;  // 2^(-1/3)
 template <int FORM = kExact>
 __device__ __forceinline__ double spline_w8(double r2, double m4h, double mk2h)
 {
-  double ir2;
-  const double d = twice_r<FORM>(r2, ir2);
+  double ir2, d;
+  if (FORM == kSingle) d = __builtin_amdgcn_sqrt(r2);
+  else d = twice_r<FORM>(r2, ir2);
   const double t = clamp01(fma(d, m4h, 1.0)), u = clamp01(fma(d, mk2h, kSplineK));
   return fma(-(u * u), u, (t * t) * t);
 }

@@ -177,8 +177,8 @@ typedef struct ccake_params {
      counterpart in the reference, which is FP64 throughout):
      0 FP64 (the reference's arithmetic);
      1 single-precision pair weights: the kernel's r and 1/r from the
-       hardware reciprocal square root alone (relative error 5.2e-8 at most),
-       without the step that refines it to FP64.  Positions, the pair
+       hardware's square root and reciprocal square root alone (relative error
+       5.2e-8 at most), without the step that refines them to FP64.  Positions, the pair
        predicate (so the pair set), the products and sums and everything
        outside the pair loops (EoS inversion, EoM, RK accumulation, shear
        update, initialisation, diffusion sums) are FP64. */
