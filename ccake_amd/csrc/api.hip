@@ -1121,6 +1121,13 @@ int ccake_initial_smoothing(ccake_event* ev)
   if (!ev) return CCAKE_ERR_INVALID;
   if (ev->init_phase < 2) { set_error("initialize_entropy_and_charge_densities first"); return CCAKE_ERR_INVALID; }
   int rc;
+  // the form of the mixed-precision pair sums, before the first of them (a small event's passes are short either way)
+  ev->many_neighbours = false;
+  if (ev->p.pair_precision == 1 && ev->p.dim == 2 && ev->nev <= 1 && ev->n >= 65536) {
+    int64_t pairs = 0;                                      // of the neighbour list, counted when it was built
+    if ((rc = ccake_last_pair_count(ev, &pairs))) return rc;
+    ev->many_neighbours = pairs >= (int64_t)kManyNeighbours * ev->n;
+  }
   if ((rc = launch_stage_begin(ev))) return rc;             // calculate_gamma_and_velocities
   if ((rc = ccake_smooth_fields(ev))) return rc;            // smooth_all_particle_fields
   if ((rc = launch_init_particles(ev, 3))) return rc;       // extensive shear, bulk, set_diffusion

@@ -168,6 +168,7 @@ struct ccake_event {
   bool sort_valid = false;
   bool no_charges = false;      // every particle's charges are zero (set at initialize, cleared by uploads)
   bool no_bulk = false;         // zeta = 0 and every particle's bulk pressure zero (likewise)
+  bool many_neighbours = false; // pair_precision 1: the mean at initialize is above kManyNeighbours
   double sort_disp = 0.0;
   double skin_frac = 0.04;      // re-sort when the bound would exceed skin_frac * rc (measured best at 40k)
   // freeze-out hypersurface (particlization on): 6 snapshot sets x 33 columns

@@ -91,7 +91,7 @@ __device__ __forceinline__ void grad_walk(const double* __restrict__ cand, const
     });
   });
   if (!KEEP) {
-    const double h2 = (FORM == kSingle ? -4.0 / ((1.0 + kRsqMean) * (1.0 + kRsqMean)) : -1.0) / m2h;   // of 1/r, too
+    const double h2 = FORM == kSingle ? -4.0 * m2h / hinv2 : -1.0 / m2h;   // kSingle: 4 h, over 1/r's mean error
     #pragma unroll
     for (int q = 0; q < NW; ++q) acc[q] *= h2;
   }
@@ -191,7 +191,8 @@ int launch_grad_pairs(ccake_event* ev)
   const double h = ev->p.hT;
   const double rc = 2.0 * h;
   const bool single = ev->p.pair_precision == 1;
-  const double hinv2 = 1.0 / (h * h), m4h = (single ? -0.5 / (1.0 + kRsqMean) : -0.25) / h, m2h = 2.0 * m4h;
+  const double hinv2 = 1.0 / (h * h), mean = ev->many_neighbours ? kRsqMean : 0.0;
+  const double m4h = (single ? -0.5 / (1.0 + mean) : -0.25) / h, m2h = 2.0 * m4h;
   const int ntiles = (n + kTile - 1) / kTile;
   const double rcs = search_radius(ev);
   const int W = grad_tile_waves(lds_slices(ev), ntiles, ev->dev->simds);

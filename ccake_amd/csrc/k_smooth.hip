@@ -394,7 +394,8 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
   const bool single = mode == 0 && ev->p.pair_precision == 1;
   const bool keep = !single && W >= kKeepSmoothWaves && keep_order(ev);
   const double hinv2 = 1.0 / (ev->p.hT * ev->p.hT);
-  const double m4h = (single ? -0.5 / (1.0 + kSqrtMean) : -0.25) / ev->p.hT, mk2h = 2.0 * kSplineK * m4h;
+  const bool root = single && W == 8 && ev->many_neighbours;
+  const double m4h = (root ? -0.5 / (1.0 + kSqrtMean) : (single ? -0.5 : -0.25)) / ev->p.hT, mk2h = 2.0 * kSplineK * m4h;
   if (W) {
     // the tile's slices reduced in LDS: the sum pass sees one slice
     ev->smooth_sum_slices = 1;
@@ -406,11 +407,12 @@ int launch_smooth_pairs(ccake_event* ev, int mode, bool count_pairs)
       constexpr int V = decltype(w)::value, FM = decltype(f)::value;
       if (m == 3) go(k_smooth_tile<3, V, FM>, V);
       else if (m == 0) go(k_smooth_tile<0, V, FM>, V);
-      else if constexpr (FM != kSingle) go(k_smooth_tile<1, V, FM>, V);
+      else if constexpr (FM != kSingle && FM != kRoot) go(k_smooth_tile<1, V, FM>, V);
     };
     const std::integral_constant<int, 8> w8;
     const std::integral_constant<int, 4> w4;
     if (keep) form(std::integral_constant<int, kKeepSmoothWaves>(), std::integral_constant<int, kKeep>());
+    else if (root) form(w8, std::integral_constant<int, kRoot>());
     else if (single && W == 8) form(w8, std::integral_constant<int, kSingle>());
     else if (single) form(w4, std::integral_constant<int, kSingle>());
     else if (W == 8 && small_event(ev, ntiles)) form(w8, std::integral_constant<int, kSmall>());

@@ -497,23 +497,33 @@ constexpr double kSplineW = 8.0;                     // spline_w / spline_w8
 __device__ __forceinline__ double clamp01(double v) { return fmin(fmax(v, 0.0), 1.0); }
 // FORM of a walk: kExact with the arithmetic above; kKeep with that of
 // q_and_inverse, spline_w and spline_g (keep_order); kSingle without the
-// Newton step (pair_precision 1): r and 1/r instead of 2 r and 2 / r, from y and
-// f as they are (v_rsq_f64: relative error 5.2e-8 at most, 1.0e-8 rms over 4M
-// arguments, less than one rounding to single precision) or, where 1/r is not
-// needed, r from v_sqrt_f64 (2.7e-8 and 8.4e-9), which takes 0 as it is;
+// Newton step (pair_precision 1): y and f as they are, so r and 1/r instead of
+// 2 r and 2 / r, with v_rsq_f64's relative error (5.2e-8 at most, 1.0e-8
+// rms over 4M arguments: less than one rounding to single precision),
 // everything else in FP64.  Single-precision arithmetic would not be faster: it
-// issues at the FP64 rate here.  188,250 particles: smoothing 612 us in FP64, 547
-// (580 with r from v_rsq_f64), gradients 970 and 910 (pair terms in FP32 with
-// compensated sums: 548 and 990); 751,500: 8.0 and 7.1 ms (7.6; 7.2), 13.0 and
-// 12.1 (12.6).  The constants m4h and m2h (mk2h) are then twice as large, and the
-// gradient's final factor.  What does not average out over the pairs, the errors'
-// mean with the weight that a pair's r has in a density or a gradient, is taken
-// out by the constants: it is -3.3e-9 for v_sqrt_f64 (-3.1e-9 to -3.5e-9 for h
-// from 0.1 to 1) and 3.3e-9 for v_rsq_f64 (2.5e-9 to 4.0e-9), as measured.
-constexpr double kSqrtMean = -3.3e-9, kRsqMean = 3.3e-9;
+// issues at the FP64 rate here.  188,250 particles: smoothing 615 -> 580 us,
+// gradients 970 -> 915 us (pair terms in FP32 with compensated sums: 548 and 990).
+// The constants m4h and m2h (mk2h) are then twice as large, and the gradient's
+// final factor.  kRoot: kSingle with r from v_sqrt_f64 where 1/r is not needed
+// (many_neighbours): two instructions fewer, 188,250 particles 547 us.
 // kSmall: kExact with the rows of a tile as one segment where that reaches less
 // (for_segments), for events whose waves do not fill the SIMDs.
-enum Form { kExact, kKeep, kSingle, kSmall };
+enum Form { kExact, kKeep, kSingle, kSmall, kRoot };
+// kRoot's rule.  v_sqrt_f64 is as exact as v_rsq_f64 (2.7e-8 and 8.4e-9), but
+// with its other errors the densities' are no longer the gradients', and where a
+// lattice has few distances (v - v_a) grad W / sigma loses by that: a stage at 402
+// neighbours has grad v off by 7.8e-9 instead of 5.4e-10.  They average out over
+// many, and then what is left, the errors' mean with the weight that a pair's r
+// has in a density or a gradient, is taken out by the constants: -3.3e-9 for
+// v_sqrt_f64 (-3.1e-9 to -3.5e-9 for h from 0.1 to 1), 3.3e-9 for v_rsq_f64
+// (2.5e-9 to 4.0e-9), as measured.  2,141 to 10,343 neighbours: sigma off by 1.9e-10
+// to 1.3e-9 (kSingle 5.2e-9 to 6.9e-9), grad p 4.6e-10 to 2.1e-9 (6.3e-9 to 8.9e-9),
+// grad v 4.8e-10 to 2.2e-9 (4.5e-10 to 2.2e-9).  So above 2,000, where smoothing is
+// most of a step besides: 751,500 particles (10,326 neighbours) 7.6 -> 7.1 ms (8.0 in
+// FP64, 7.2 with FP32 terms), gradients 12.2 (13.0; 12.6).  An event alone: a
+// batch's mean says little of its events.
+constexpr double kSqrtMean = -3.3e-9, kRsqMean = 3.3e-9;
+constexpr int kManyNeighbours = 2000;
 // 2 r of a pair; ir2 receives 2 / r (kSingle: r and 1 / r)
 template <int FORM>
 __device__ __forceinline__ double twice_r(double r2, double& ir2)
@@ -544,7 +554,7 @@ template <int FORM = kExact>
 __device__ __forceinline__ double spline_w8(double r2, double m4h, double mk2h)
 {
   double ir2, d;
-  if (FORM == kSingle) d = __builtin_amdgcn_sqrt(r2);
+  if (FORM == kRoot) d = __builtin_amdgcn_sqrt(r2);
   else d = twice_r<FORM>(r2, ir2);
   const double t = clamp01(fma(d, m4h, 1.0)), u = clamp01(fma(d, mk2h, kSplineK));
   return fma(-(u * u), u, (t * t) * t);

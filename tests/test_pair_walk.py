@@ -128,6 +128,32 @@ def test_single_precision_weights(dev, slices, shear):
         assert 0.0 < err <= (5.2e-8 if f == "SIGMA_LAB" else 2e-6), (f, err)
 
 
+# above 2,000 neighbours r comes from the square root instruction (2.7e-8 at most,
+# at twice which a pair's weight can be off) and the errors' mean is taken out: of
+# -3.3e-9 in r, so 6.6e-9 in a density, no more than 2e-9 is left
+def test_single_precision_weights_of_many_neighbours(dev):
+    d = cloud(66000, 2.4)
+    cfg = config.base_params(t0=0.6, dt=0.01, particlization=0, eta_mode=config.ETA_CONSTANT, constant_eta_over_s=0.08,
+                             cells_per_rc=4, x_subcells=4)
+    eos = ccake_amd.Eos(dev, 0, 0.75)
+    got = []
+    for pp in (0, 1):
+        ev = ccake_amd.Event(dev, eos, dict(cfg, pair_precision=pp), len(d["x"]))
+        ccake_amd.load_event(ev, d)
+        ev.initialize()
+        ev.get_time_derivatives()
+        got.append({f: ev.download(ccake_amd.FIELDS["CCAKE_F_" + f]) for f in ("SIGMA_LAB", "S", "GRADP0", "GRADE0", "GRADV0")})
+        got[-1]["BTRACK"] = ev.download_int("CCAKE_I_BTRACK")
+        ev.close()
+    eos.close()
+    assert np.array_equal(got[0]["BTRACK"], got[1].pop("BTRACK")) and np.mean(got[0].pop("BTRACK")) >= 2000
+    for f, a in got[0].items():
+        err = np.max(np.abs(got[1][f] - a)) / np.max(np.abs(a))
+        print(f, err)
+        assert 0.0 < err <= (5.4e-8 if f in ("SIGMA_LAB", "S") else 2e-6), (f, err)
+    assert abs(np.mean(got[1]["SIGMA_LAB"] / got[0]["SIGMA_LAB"] - 1.0)) <= 2e-9
+
+
 # An event for which one slice of partial sums is set aside (262,144 particles
 # are 4,096 tiles: whole rounds of the chip's SIMDs) runs its tiles of 8 waves in
 # no more device memory: the diffusion pass, which stores every slice's sums,
