@@ -65,10 +65,9 @@ def test_batch_equals_alone(dev, table_eos, precision):
     """Three lumpy viscous BSQ events of 8,077, 3,345 and 5,746 particles on
     the table EoS (0.1 fm lattice, different seeds and widths): after
     initialization and 20 steps in one batch every event's fields are within
-    1e-12 (whole-field relative; FP64 pair sums; measured 4e-14) or 1e-6
-    (mixed precision: the slices' FP32 blocks begin at other candidates, so
-    the batch and the run alone differ by FP32 rounding, 2.5e-8 measured) of
-    the same event run alone, with equal btrack and per-event entropy."""
+    1e-12 (whole-field relative, in either precision: a pair's weight is the
+    same in the batch, and the sums are FP64; measured 5e-14) of the same
+    event run alone, with equal btrack and per-event entropy."""
     cfg = dict(config.lumpy_params(), pair_precision=precision)
     ics = three_events(0.1)
     b, alone = make(dev, table_eos, cfg, ics)
@@ -76,7 +75,7 @@ def test_batch_equals_alone(dev, table_eos, precision):
     b.run_steps(cfg["dt"], 20)
     for ev in alone:
         ev.run_steps(cfg["dt"], 20)
-    tol = 1e-12 if precision == 0 else 1e-6
+    tol = 1e-12
     s_batch = b.batch_reduce("CCAKE_R_ENTROPY")
     worst = 0.0
     for e, ev in enumerate(alone):
@@ -87,7 +86,7 @@ def test_batch_equals_alone(dev, table_eos, precision):
             err = whole(b.download(fid(lab))[sl], ev.download(fid(lab)))
             worst = max(worst, err)
             assert err <= tol, (e, lab, err)
-        assert abs(s_batch[e] / ev.reduce("CCAKE_R_ENTROPY") - 1.0) < (1e-13 if precision == 0 else 1e-9)
+        assert abs(s_batch[e] / ev.reduce("CCAKE_R_ENTROPY") - 1.0) < 1e-13
     print(f"precision {precision}: worst field difference batch vs alone {worst:.2e}", flush=True)
     b.close()
     for ev in alone:
