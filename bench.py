@@ -47,21 +47,22 @@ if ROOT not in sys.path:
 PEAK_HBM_GBS = 8000.0
 PEAK_FP64_TFLOPS = 78.6
 
-# Algorithmic work per unit, FMA = 2 flop, sqrt/div = 1 (frozen constants),
-# per launched variant of the pair kernels.
-# Smoothing, per directed pair: distance 5, sqrt 1, q 1, W 7, sigma_lab
-# m W (2), then m ext W (3) for each of s, rho_B, rho_S, rho_Q: 28; the
-# charge-free variant (k_smooth_slice<3>, an event without charges) 19.
-FLOP_PER_PAIR_SMOOTH = {True: 28, False: 19}               # charges on / off
-# Gradients, per directed pair (2D): 95 with shear on, 62 with it off; the
-# bulk-free variant (no grad Pi sums: an ideal fluid with zeta = 0) skips 4.
-FLOP_PER_PAIR_GRAD = {(True, True): 95, (True, False): 91, (False, True): 62, (False, False): 58}
-# 3+1D (D = 3, isotropic kernel), per directed pair: smoothing 37 (offsets 3,
-# distance 5, q and 1/q 9, spline 10, five accumulations 10); gradients 99
-# with shear on (offsets 3, distance 5, q and 1/q 9, spline gradient 9,
-# weight 4, 21 accumulations 39, shear 30), 69 with it off.
-FLOP_PER_PAIR_SMOOTH3 = 37
-FLOP_PER_PAIR_GRAD3 = {True: 99, False: 69}
+# Work per directed pair of the pair kernels in the arithmetic they do, an FMA
+# as 2 flop, a reciprocal square root as 1 (the FP64 instruction counters of
+# profiles/pmc_valu_lumpy_200k.md give the same per candidate).
+# Smoothing: offsets and r^2 5, r 6 (the guard against 0, the reciprocal square
+# root, one Newton step), W 9, sigma_lab, s, rho_B, rho_S and rho_Q 2 each: 30; the
+# charge-free variant (an event without charges) has two sums: 24.
+FLOP_PER_PAIR_SMOOTH = {True: 30, False: 24}               # charges on / off
+# Gradients (2D): offsets and r^2 5, r and 1/r 7, grad W 11, 20 sums with shear on
+# (63), 12 with it off (47); the bulk-free variant (no grad Pi sums: an ideal
+# fluid with zeta = 0) has two fewer.
+FLOP_PER_PAIR_GRAD = {(True, True): 63, (True, False): 59, (False, True): 47, (False, False): 43}
+# 3+1D (D = 3, isotropic kernel): smoothing 33 (offsets and r^2 8, r 6, W 9, five
+# sums 10); gradients 27 (offsets and r^2 8, r and 1/r 7, grad W 12) and 39 sums
+# with shear on (105), 21 with it off (69).
+FLOP_PER_PAIR_SMOOTH3 = 33
+FLOP_PER_PAIR_GRAD3 = {True: 105, False: 69}
 
 
 def parse():
