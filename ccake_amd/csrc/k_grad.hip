@@ -24,8 +24,8 @@ namespace ccake {
 // BULK false: the event's bulk pressure is zero on every particle (zeta = 0
 // and no initial bulk, checked at initialize), so the grad Pi sums are the
 // exact zeros the full walk would give and are not accumulated.
-// Bound: the FP64 vector unit (80 % busy), 38 instructions per candidate and
-// wave: the 20 sums, 5 for the offsets and r^2, 13 for the kernel.  FP64
+// Bound: the FP64 vector unit (80 % busy), 39 instructions per candidate and
+// wave: the 20 sums, 5 for the offsets and r^2, 14 for the kernel.  FP64
 // matrix instructions run in the same unit at the same rate (16x16x4: 65
 // cycles, a vector instruction 4), so the sums stay on the vector side.
 // 188,250 particles (479M pairs): 1.30 ms per launch with 50 instructions
