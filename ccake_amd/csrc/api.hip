@@ -530,9 +530,14 @@ int ccake_eos_create(ccake_dev* dev, const ccake_eos_desc* desc, ccake_eos** out
     t.ginv[a] = (t.dims[a] <= 1 || std::fabs(t.gdel[a]) < 1e-30) ? 0.0 : 1.0 / t.gdel[a];
     t.mins[a] = desc->mins[a]; t.maxs[a] = desc->maxs[a];
   }
-  e->h_tab = new double[nn * 17];
+  // A cell's second corner along an axis of one node has the weight 0, and its
+  // value is read: zeros past the table's end, as far as those corners reach.
+  size_t room = nn;
+  for (size_t a = 4, stride = 1; a-- > 0; stride *= (size_t)t.dims[a]) if (t.dims[a] <= 1) room += stride;
+  e->h_tab = new double[room * 17];
   std::memcpy(e->h_tab, desc->table, nn * 17 * sizeof(double));
-  std::vector<double> t5(nn * 5);
+  std::fill(e->h_tab + nn * 17, e->h_tab + room * 17, 0.0);
+  std::vector<double> t5(room * 5);
   for (int q = 0; q < 5; ++q) { t.dmin[q] = INFINITY; t.dmax[q] = -INFINITY; }
   bool finite = true;
   for (size_t k = 0; k < nn; ++k) {
@@ -547,7 +552,7 @@ int ccake_eos_create(ccake_dev* dev, const ccake_eos_desc* desc, ccake_eos** out
     }
   }
   if (!finite) for (int q = 0; q < 5; ++q) { t.dmin[q] = 1.0; t.dmax[q] = 0.0; }   // no bounds: never skipped
-  e->bytes = nn * 22 * sizeof(double);
+  e->bytes = room * 22 * sizeof(double);
   {
     std::lock_guard<std::mutex> lk(dev->mu);
     if (dev->budget && dev->used + e->bytes > dev->budget) {
@@ -569,11 +574,11 @@ int ccake_eos_create(ccake_dev* dev, const ccake_eos_desc* desc, ccake_eos** out
       return hip_fail(err, what);
     };
     hipError_t err;
-    if ((err = hipMalloc((void**)&e->d_tab, nn * 17 * sizeof(double))) != hipSuccess) return fail(err, "hipMalloc(table)");
-    if ((err = hipMalloc((void**)&e->d_tab4, nn * 5 * sizeof(double))) != hipSuccess) return fail(err, "hipMalloc(table)");
-    if ((err = hipMemcpy(e->d_tab, desc->table, nn * 17 * sizeof(double), hipMemcpyHostToDevice)) != hipSuccess)
+    if ((err = hipMalloc((void**)&e->d_tab, room * 17 * sizeof(double))) != hipSuccess) return fail(err, "hipMalloc(table)");
+    if ((err = hipMalloc((void**)&e->d_tab4, room * 5 * sizeof(double))) != hipSuccess) return fail(err, "hipMalloc(table)");
+    if ((err = hipMemcpy(e->d_tab, e->h_tab, room * 17 * sizeof(double), hipMemcpyHostToDevice)) != hipSuccess)
       return fail(err, "hipMemcpy(table)");
-    if ((err = hipMemcpy(e->d_tab4, t5.data(), nn * 5 * sizeof(double), hipMemcpyHostToDevice)) != hipSuccess)
+    if ((err = hipMemcpy(e->d_tab4, t5.data(), room * 5 * sizeof(double), hipMemcpyHostToDevice)) != hipSuccess)
       return fail(err, "hipMemcpy(table)");
   }
   ch.tab = e->d_tab;

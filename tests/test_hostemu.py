@@ -117,6 +117,18 @@ def test_slice_counts(emu_lib):
     assert r.stdout.rstrip().endswith("OK")
 
 
+def test_table_axes_of_one_node(emu_lib):
+    """EoS tables with one node along some axes, under AddressSanitizer: no
+    read past the table, on the host or by the kernels, and the table's own
+    values at its nodes."""
+    env = dict(os.environ)
+    r = subprocess.run(["bash", os.path.join(EMU, "emu.sh"), os.path.join(EMU, "run_one_node_axis.py")],
+                       capture_output=True, text=True, timeout=600, env=env)
+    print(r.stdout[-4000:], r.stderr[-8000:])
+    assert r.returncode == 0 and "AddressSanitizer" not in r.stderr
+    assert r.stdout.rstrip().endswith("OK")
+
+
 def test_private_columns_disjoint():
     """Every multi-column private member owns its columns (the overlap that
     wrote past the field buffer is gone): parse the enumeration and check
